@@ -111,7 +111,7 @@ typedef struct vrx_bvh {
   void *d_leaves;         /* n * leaf record (48/16/32/0/32/32 B: tri/sphere/cyl/box/cone/curve) */
   uint32_t *d_leaf_ids;   /* n: sorted leaf -> original primitive index */
   void *d_header;         /* 64 B: root box (6 f32), height, root, n, type */
-  void *d_wide;           /* optional (n-1) * 128 B 4-wide nodes (vrx_bvh_widen), or NULL */
+  void *d_wide;           /* optional 4-wide nodes (vrx_bvh_widen or vrx_bvh_pack), or NULL */
 } vrx_bvh;
 
 typedef struct vrx_bvh_sizes {
@@ -129,6 +129,14 @@ int vrx_bvh_build(const vrx_prims *prims, const vrx_bvh *out, void *d_workspace,
  * and root.  Writes bvh->d_wide, which must hold vrx_bvh_wide_bytes(n). */
 size_t vrx_bvh_wide_bytes(uint32_t n);
 int vrx_bvh_widen(const vrx_bvh *bvh, uint32_t n, vrx_stream s);
+/* The same 4-wide tree in 64-byte records: child boxes as 8-bit steps on a
+ * grid over the record's box, rounded outwards; the traversal checks a hit
+ * against its exact leaf box, so frames do not depend on the node format.
+ * Writes bvh->d_wide, which must hold vrx_bvh_packed_bytes(type, n); type is
+ * the primitive type of the build (VRX_BOX: the instance level, which also
+ * stores its n entry boxes). */
+size_t vrx_bvh_packed_bytes(int32_t type, uint32_t n);
+int vrx_bvh_pack(const vrx_bvh *bvh, int32_t type, uint32_t n, vrx_stream s);
 /* Debug/parity hooks: read back the sorted Morton codes (n) and the order. */
 int vrx_bvh_build_debug(const vrx_prims *prims, const vrx_bvh *out, void *d_workspace,
     size_t workspace_bytes, uint32_t *d_codes_out, float *d_cbox_out, vrx_stream s);
@@ -233,8 +241,10 @@ typedef struct vrx_scene {
   uint32_t num_lights;
   const vrx_light *d_lights;    /* device array (directLight renderer) */
   uint32_t num_majorant_grids;  /* volumes that carry d_majorant */
-  uint32_t pad;
+  uint32_t wide_format;         /* with wide: VRX_WIDE_PACKED = every d_wide was written by
+                                   vrx_bvh_pack; any other value = by vrx_bvh_widen */
 } vrx_scene;
+#define VRX_WIDE_PACKED 0x34503634u
 
 typedef struct vrx_camera {
   float pos[3];

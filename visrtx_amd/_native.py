@@ -83,7 +83,7 @@ class vrx_scene(C.Structure):
                 ("num_volumes", C.c_uint32), ("single_type", C.c_int32),
                 ("max_volume_voxels", C.c_uint64), ("wide", C.c_uint32),
                 ("num_lights", C.c_uint32), ("d_lights", C.c_void_p),
-                ("num_majorant_grids", C.c_uint32), ("pad", C.c_uint32)]
+                ("num_majorant_grids", C.c_uint32), ("wide_format", C.c_uint32)]
 
 
 class vrx_volume(C.Structure):
@@ -174,6 +174,8 @@ def hip() -> C.CDLL:
             "vrx_bvh_build_debug": (i32, [vp, vp, vp, sz, vp, vp, vp]),
             "vrx_bvh_wide_bytes": (sz, [u32]),
             "vrx_bvh_widen": (i32, [vp, u32, vp]),
+            "vrx_bvh_packed_bytes": (sz, [i32, u32]),
+            "vrx_bvh_pack": (i32, [vp, i32, u32, vp]),
             "vrx_render_scratch_bytes": (sz, [vp, vp, u32, u32]),
             "vrx_frame_clear": (i32, [vp, vp]),
             "vrx_render": (i32, [vp, vp, vp, vp, vp]),

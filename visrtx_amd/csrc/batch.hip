@@ -33,7 +33,7 @@ __device__ __forceinline__ vrx_camera load_camera(const vrx_camera *cams, uint32
   return c;
 }
 
-template <int PT, bool TWO, bool WIDE, int KIND>
+template <int PT, bool TWO, int WIDE, int KIND>
 __device__ __forceinline__ void render_batch(const vrx_scene &sc, const vrx_renderer &r,
     const vrx_batch &b, uint32_t sd, uint32_t cap, uint32_t *spill, uint32_t tiles_x,
     uint32_t tiles_y)
@@ -88,7 +88,7 @@ __device__ __forceinline__ void render_batch(const vrx_scene &sc, const vrx_rend
   }
 }
 
-template <int PT, bool TWO, bool WIDE, int KIND>
+template <int PT, bool TWO, int WIDE, int KIND>
 __global__ __launch_bounds__(kBatchMaxBlock) void k_render_batch(vrx_scene sc, vrx_renderer r,
     vrx_batch b, uint32_t sd, uint32_t cap, uint32_t *spill, uint32_t tiles_x, uint32_t tiles_y)
 {
@@ -100,7 +100,7 @@ __global__ __launch_bounds__(kBatchMaxBlock) void k_render_batch(vrx_scene sc, v
 // of the scene), and on the 64-view scene the fifth wave outweighs the few
 // registers it spills (14.8 -> 13.6 ms).  AO and directLight would spill
 // 160-320 B per lane and keep the unconstrained kernel.
-template <int PT, bool TWO, bool WIDE>
+template <int PT, bool TWO, int WIDE>
 __global__ __launch_bounds__(kBatchMaxBlock) __attribute__((amdgpu_waves_per_eu(5, 8))) void
 k_render_batch_raycast(vrx_scene sc, vrx_renderer r, vrx_batch b, uint32_t sd, uint32_t cap,
     uint32_t *spill, uint32_t tiles_x, uint32_t tiles_y)
@@ -131,7 +131,7 @@ static uint32_t cap_for(const vrx_scene &sc, uint32_t sd, bool wide)
   return m > sd ? m - sd : 0u;
 }
 
-template <int PT, bool WIDE, int KIND>
+template <int PT, int WIDE, int KIND>
 static const void *kernel_ptr_k(bool two)
 {
   if constexpr (KIND == VRX_RENDER_RAYCAST && PT >= 0)
@@ -142,7 +142,7 @@ static const void *kernel_ptr_k(bool two)
                : (const void *)&k_render_batch<PT, false, WIDE, KIND>;
 }
 
-template <int PT, bool WIDE>
+template <int PT, int WIDE>
 static const void *kernel_ptr(bool two, int kind)
 {
   if (kind == VRX_RENDER_AO)
@@ -152,7 +152,7 @@ static const void *kernel_ptr(bool two, int kind)
   return kernel_ptr_k<PT, WIDE, VRX_RENDER_RAYCAST>(two);
 }
 
-template <bool WIDE>
+template <int WIDE>
 static const void *pick_kernel_w(const vrx_scene &sc, int kind)
 {
   const bool two = sc.num_entries > 1;
@@ -170,7 +170,8 @@ static const void *pick_kernel_w(const vrx_scene &sc, int kind)
 
 static const void *pick_kernel(const vrx_scene &sc, bool wide, int kind)
 {
-  return wide ? pick_kernel_w<true>(sc, kind) : pick_kernel_w<false>(sc, kind);
+  return !wide ? pick_kernel_w<0>(sc, kind)
+      : sc.wide_format == VRX_WIDE_PACKED ? pick_kernel_w<2>(sc, kind) : pick_kernel_w<1>(sc, kind);
 }
 
 __global__ void k_reset_counter(uint32_t *c)

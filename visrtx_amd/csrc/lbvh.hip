@@ -673,45 +673,6 @@ __device__ __forceinline__ void write_leaf(
   }
 }
 
-// float4s per leaf record
-template <int T>
-constexpr int record_quads()
-{
-  return T == VRX_SPHERE ? 1
-      : (T == VRX_CYLINDER || T == VRX_CONE || T == VRX_CURVE) ? 2 : (T == VRX_TRIANGLE ? 3 : 0);
-}
-
-// box of a leaf record (same bounds rule as prim_box)
-template <int T>
-__device__ __forceinline__ void record_box(const float4 *L, v3 &lo, v3 &hi)
-{
-  if constexpr (T == VRX_SPHERE) {
-    const float4 a = L[0];
-    lo = mk(a.x - a.w, a.y - a.w, a.z - a.w);
-    hi = mk(a.x + a.w, a.y + a.w, a.z + a.w);
-  } else if constexpr (T == VRX_CYLINDER) {
-    const float4 a = L[0], b = L[1];
-    v3 mn = vmin(mk(a.x, a.y, a.z), mk(b.x, b.y, b.z)), mx = vmax(mk(a.x, a.y, a.z), mk(b.x, b.y, b.z));
-    lo = mk(mn.x - a.w, mn.y - a.w, mn.z - a.w);
-    hi = mk(mx.x + a.w, mx.y + a.w, mx.z + a.w);
-  } else if constexpr (T == VRX_CONE) {
-    const float4 a = L[0], b = L[1];
-    v3 mn = vmin(mk(a.x, a.y, a.z), mk(b.x, b.y, b.z)), mx = vmax(mk(a.x, a.y, a.z), mk(b.x, b.y, b.z));
-    float r = fmaxf(a.w, b.w);
-    lo = mk(mn.x - r, mn.y - r, mn.z - r);
-    hi = mk(mx.x + r, mx.y + r, mx.z + r);
-  } else if constexpr (T == VRX_CURVE) {
-    const float4 a = L[0], b = L[1];
-    lo = vmin(mk(a.x - a.w, a.y - a.w, a.z - a.w), mk(b.x - b.w, b.y - b.w, b.z - b.w));
-    hi = vmax(mk(a.x + a.w, a.y + a.w, a.z + a.w), mk(b.x + b.w, b.y + b.w, b.z + b.w));
-  } else if constexpr (T == VRX_TRIANGLE) {
-    const float4 a = L[0], b = L[1], c = L[2];
-    v3 v0 = mk(a.x, a.y, a.z), v1 = mk(b.x, b.y, b.z), v2 = mk(c.x, c.y, c.z);
-    lo = vmin(vmin(v0, v1), v2);
-    hi = vmax(vmax(v0, v1), v2);
-  }
-}
-
 // box of sorted leaf k, from its leaf record
 template <int T>
 __device__ __forceinline__ void leaf_box(
@@ -1250,6 +1211,149 @@ __global__ __launch_bounds__(256) void k_widen(const Node *nodes, uint32_t ninne
     gst(out, q, s_rec[q]);
 }
 
+// --------------------------------------------------------------------------
+// packed 4-wide nodes
+// --------------------------------------------------------------------------
+// Packed record i from BVH2 node i: its grandchildren, a leaf child keeping
+// its slot; where that leaves a slot free, the inner child with the largest
+// box is opened once more.  An inner child of a record is therefore at least
+// two BVH2 levels below it, so a walk pushes as many entries as over the
+// 128-byte records.
+//
+// Per axis the grid starts 1.5 steps below the record's box, a step being
+// 1/250 of its extent, but no less than 2^-22 of the box's largest coordinate
+// (about two ulps, so that the origin, rounded to fp32, stays within half a
+// step) and 1e-20.  Planes are rounded outwards in FP64.  A record whose box
+// is not finite gets a NaN origin: every plane distance is then NaN, which
+// the slab test's min / max drop, and all its children are visited.
+struct PackSlot {
+  float b[6];
+  uint32_t link;
+};
+
+__device__ __forceinline__ float slot_area(const PackSlot &s)
+{
+  const float x = s.b[3] - s.b[0], y = s.b[4] - s.b[1], z = s.b[5] - s.b[2];
+  return (s.link & kLeafBit) ? -1.0f : x * y + (y * z + z * x);
+}
+
+// packed bytes of the axis `a` of four slots; false if the axis has no finite grid
+__device__ __forceinline__ bool pack_axis(const PackSlot s[4], uint32_t cnt, int a, float &org,
+    float &scale, uint32_t &lo, uint32_t &hi)
+{
+  double mn = INFINITY, mx = -INFINITY;
+  bool fin = true;
+#pragma unroll
+  for (int c = 0; c < 4; c++) {
+    if ((uint32_t)c < cnt) {
+      // a box of negative extent (a negative radius) is tested as its mirror
+      const double p = s[c].b[a], q = s[c].b[3 + a];
+      fin = fin && p - p == 0.0 && q - q == 0.0;
+      mn = fmin(mn, fmin(p, q));
+      mx = fmax(mx, fmax(p, q));
+    }
+  }
+  const double big = fmax(fabs(mn), fabs(mx));
+  const float st = (float)fmax(fmax((mx - mn) * (1.0 / 250.0), big * 0x1p-22), 1e-20);
+  const float og = (float)(mn - 1.5 * (double)st);
+  fin = fin && st < 1e36f && og - og == 0.0f;
+  lo = hi = 0u;
+#pragma unroll
+  for (int c = 0; c < 4; c++) {
+    uint32_t ql = 255u, qh = 0u;
+    if ((uint32_t)c < cnt) {
+      const double p = s[c].b[a], q = s[c].b[3 + a];
+      const double l = floor((fmin(p, q) - (double)og) / (double)st - kPackMargin);
+      const double h = ceil((fmax(p, q) - (double)og) / (double)st + kPackMargin);
+      fin = fin && l >= 0.0 && h <= 255.0;
+      ql = fin ? (uint32_t)l : 0u;
+      qh = fin ? (uint32_t)h : 255u;
+    }
+    lo |= ql << (8 * c);
+    hi |= qh << (8 * c);
+  }
+  scale = fin ? st : 1.0f;
+  org = fin ? og : NAN;
+  return fin;
+}
+
+// LEAF_BOX: also store the exact box of every leaf by its primitive (the
+// instance level: entry boxes, which have no leaf record to derive them from)
+template <bool LEAF_BOX>
+__global__ __launch_bounds__(256) void k_pack(const Node *nodes, uint32_t ninner, Node4p *out,
+    const uint32_t *leaf_ids, float *leaf_box)
+{
+  const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= ninner)
+    return;
+  PackSlot s[4];
+  const Node nd = gld_node(nodes, i);
+  node_child(nd, 0, s[0].b, s[0].link);
+  node_child(nd, 1, s[1].b, s[1].link);
+  if constexpr (LEAF_BOX) {
+#pragma unroll
+    for (int j = 0; j < 2; j++)
+      if (s[j].link & kLeafBit) {
+        float *b = leaf_box + 6 * (size_t)gld(leaf_ids, s[j].link & ~kLeafBit);
+#pragma unroll
+        for (int q = 0; q < 6; q++)
+          gst(b, q, s[j].b[q]);
+      }
+  }
+  const bool in0 = !(s[0].link & kLeafBit), in1 = !(s[1].link & kLeafBit);
+  uint32_t cnt = 2;
+  s[2] = s[3] = s[1];
+  if (in0 && in1) {
+    const Node c1 = gld_node(nodes, s[1].link), c0 = gld_node(nodes, s[0].link);
+    node_child(c0, 0, s[0].b, s[0].link);
+    node_child(c0, 1, s[1].b, s[1].link);
+    node_child(c1, 0, s[2].b, s[2].link);
+    node_child(c1, 1, s[3].b, s[3].link);
+    cnt = 4;
+  } else if (in0 || in1) {
+    // the leaf in slot 0, the inner child's children in slots 1 and 2, and
+    // the larger inner one of those opened into slots 1, 3 or 2, 3
+    const uint32_t inner = in0 ? s[0].link : s[1].link;
+    if (in0)
+      s[0] = s[1];
+    const Node c = gld_node(nodes, inner);
+    node_child(c, 0, s[1].b, s[1].link);
+    node_child(c, 1, s[2].b, s[2].link);
+    cnt = 3;
+    const float a1 = slot_area(s[1]), a2 = slot_area(s[2]);
+    const bool first = a1 >= a2;
+    const uint32_t open = first ? s[1].link : s[2].link;
+    if (!(open & kLeafBit)) {
+      const Node g = gld_node(nodes, open);
+      PackSlot n0;
+      node_child(g, 0, n0.b, n0.link);
+      node_child(g, 1, s[3].b, s[3].link);
+      if (first)
+        s[1] = n0;
+      else
+        s[2] = n0;
+      cnt = 4;
+    }
+  }
+  Node4p r;
+  const bool fx = pack_axis(s, cnt, 0, r.ox, r.sx, r.lox, r.hix);
+  const bool fy = pack_axis(s, cnt, 1, r.oy, r.sy, r.loy, r.hiy);
+  const bool fz = pack_axis(s, cnt, 2, r.oz, r.sz, r.loz, r.hiz);
+  if (!(fx && fy && fz))
+    r.ox = r.oy = r.oz = NAN;
+  r.link.x = s[0].link;
+  r.link.y = s[1].link;
+  r.link.z = cnt > 2 ? s[2].link : kPackEmpty;
+  r.link.w = cnt > 3 ? s[3].link : kPackEmpty;
+  float4 *w = (float4 *)(out + i);
+  gst(w, 0, make_float4(r.ox, r.oy, r.oz, r.sx));
+  gst(w, 1, make_float4(r.sy, r.sz, __uint_as_float(r.lox), __uint_as_float(r.loy)));
+  gst(w, 2, make_float4(__uint_as_float(r.loz), __uint_as_float(r.hix), __uint_as_float(r.hiy),
+      __uint_as_float(r.hiz)));
+  gst(w, 3, make_float4(__uint_as_float(r.link.x), __uint_as_float(r.link.y),
+      __uint_as_float(r.link.z), __uint_as_float(r.link.w)));
+}
+
 __global__ void k_empty_header(vrx_bvh_header *h, int type)
 {
   write_header(h, mk(INFINITY, INFINITY, INFINITY), mk(-INFINITY, -INFINITY, -INFINITY), 0u,
@@ -1402,6 +1506,34 @@ int vrx_bvh_build_debug(const vrx_prims *prims, const vrx_bvh *out, void *d_work
 {
   return bvh_build_impl(
       prims, out, d_workspace, workspace_bytes, d_codes_out, d_cbox_out, (hipStream_t)s);
+}
+
+size_t vrx_bvh_packed_bytes(int32_t type, uint32_t n)
+{
+  if (n < 2)
+    return 0;
+  return (size_t)(n - 1) * sizeof(Node4p) + (type == VRX_BOX ? (size_t)n * 24 : 0);
+}
+
+int vrx_bvh_pack(const vrx_bvh *bvh, int32_t type, uint32_t n, vrx_stream s)
+{
+  VRX_ARG(bvh, "bvh");
+  VRX_ARG(type >= 0 && type <= VRX_CURVE, "type");
+  if (n < 2)
+    return VRX_OK; // a single leaf (or nothing): no inner nodes
+  VRX_ARG(bvh->d_nodes && bvh->d_wide, "bvh nodes / packed buffer");
+  VRX_ARG(type != VRX_BOX || bvh->d_leaf_ids, "leaf ids");
+  const uint32_t ninner = n - 1;
+  const dim3 grid((ninner + 255) / 256);
+  Node4p *out = (Node4p *)bvh->d_wide;
+  if (type == VRX_BOX)
+    hipLaunchKernelGGL(k_pack<true>, grid, dim3(256), 0, (hipStream_t)s,
+        (const Node *)bvh->d_nodes, ninner, out, bvh->d_leaf_ids, (float *)(out + ninner));
+  else
+    hipLaunchKernelGGL(k_pack<false>, grid, dim3(256), 0, (hipStream_t)s,
+        (const Node *)bvh->d_nodes, ninner, out, (const uint32_t *)nullptr, (float *)nullptr);
+  VRX_LAUNCH_CHECK();
+  return VRX_OK;
 }
 
 size_t vrx_bvh_wide_bytes(uint32_t n)

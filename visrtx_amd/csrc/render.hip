@@ -25,7 +25,7 @@
 
 namespace vrx {
 
-template <int PT, bool TWO, int KIND, bool WIDE, int LONG = 0>
+template <int PT, bool TWO, int KIND, int WIDE, int LONG = 0>
 __device__ __forceinline__ void render_tile(const vrx_scene &sc, const vrx_camera &cam,
     const vrx_renderer &r, const vrx_frame &f, uint32_t sd, uint32_t ovf_cap, uint32_t *scratch,
     const LongRays *lr = nullptr)
@@ -60,7 +60,7 @@ __device__ __forceinline__ void render_tile(const vrx_scene &sc, const vrx_camer
   }
 }
 
-template <int PT, bool TWO, int KIND, bool WIDE>
+template <int PT, bool TWO, int KIND, int WIDE>
 __global__ __launch_bounds__(kBlock) void k_render(vrx_scene sc, vrx_camera cam, vrx_renderer r,
     vrx_frame f, uint32_t sd, uint32_t ovf_cap, uint32_t *scratch)
 {
@@ -74,7 +74,7 @@ __global__ __launch_bounds__(kBlock) void k_render(vrx_scene sc, vrx_camera cam,
 // 13.1 -> 11.9 ms, directLight 4 spp 6.4 -> 5.7 ms; 1M instances +7 %).
 // Single-level raycast (66-88 VGPRs) and the generic kernel (130-150 VGPRs)
 // keep k_render.
-template <int PT, bool TWO, int KIND, bool WIDE>
+template <int PT, bool TWO, int KIND, int WIDE>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(6, 8))) void k_render_occ6(
     vrx_scene sc, vrx_camera cam, vrx_renderer r, vrx_frame f, uint32_t sd, uint32_t ovf_cap,
     uint32_t *scratch)
@@ -84,7 +84,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(6, 8))) 
 
 // The one-level primitive raycast with a step budget: walks longer than
 // lr.budget loop iterations queue their pixel for k_render_long.
-template <int PT, bool WIDE>
+template <int PT, int WIDE>
 __global__ __launch_bounds__(kBlock) void k_render_defer(vrx_scene sc, vrx_camera cam,
     vrx_renderer r, vrx_frame f, uint32_t sd, uint32_t ovf_cap, uint32_t *scratch, LongRays lr)
 {
@@ -94,7 +94,7 @@ __global__ __launch_bounds__(kBlock) void k_render_defer(vrx_scene sc, vrx_camer
 // The queued pixels, 16 lanes each (four per wave), over a resident grid.
 // Dynamic LDS: the lanes' private short stacks (sd entries each), then one
 // shared stack of lr.gcap entries per lane group.
-template <int PT, bool WIDE>
+template <int PT, int WIDE>
 __global__ __launch_bounds__(kBlock) void k_render_long(vrx_scene sc, vrx_camera cam,
     vrx_renderer r, vrx_frame f, uint32_t sd, uint32_t ovf_cap, uint32_t *scratch, LongRays lr)
 {
@@ -653,7 +653,7 @@ static size_t long_queue_offset(uint32_t width, uint32_t height, uint32_t cap)
   return 256 + tiles * kBlock * (size_t)cap * 4;
 }
 
-template <int PT, bool TWO, int KIND, bool WIDE>
+template <int PT, bool TWO, int KIND, int WIDE>
 static void launch_one(const vrx_scene &sc, const vrx_camera &cam, const vrx_renderer &r,
     const vrx_frame &f, uint32_t sd, uint32_t cap, hipStream_t s)
 {
@@ -698,7 +698,7 @@ static void launch_one(const vrx_scene &sc, const vrx_camera &cam, const vrx_ren
         sd, cap, (uint32_t *)f.d_scratch);
 }
 
-template <int PT, bool TWO, bool WIDE>
+template <int PT, bool TWO, int WIDE>
 static void launch_kw(const vrx_scene &sc, const vrx_camera &cam, const vrx_renderer &r,
     const vrx_frame &f, uint32_t sd, uint32_t cap, hipStream_t s)
 {
@@ -714,10 +714,12 @@ template <int PT, bool TWO>
 static int launch_kind(const vrx_scene &sc, const vrx_camera &cam, const vrx_renderer &r,
     const vrx_frame &f, uint32_t sd, uint32_t cap, hipStream_t s)
 {
-  if (wide_of(&r))
-    launch_kw<PT, TWO, true>(sc, cam, r, f, sd, cap, s);
+  if (wide_of(&r) && sc.wide_format == VRX_WIDE_PACKED)
+    launch_kw<PT, TWO, 2>(sc, cam, r, f, sd, cap, s);
+  else if (wide_of(&r))
+    launch_kw<PT, TWO, 1>(sc, cam, r, f, sd, cap, s);
   else
-    launch_kw<PT, TWO, false>(sc, cam, r, f, sd, cap, s);
+    launch_kw<PT, TWO, 0>(sc, cam, r, f, sd, cap, s);
   VRX_LAUNCH_CHECK();
   return VRX_OK;
 }
@@ -774,7 +776,7 @@ int vrx_render(const vrx_scene *scene, const vrx_camera *cam, const vrx_renderer
   VRX_ARG(r->node_width == 0 || r->node_width == 2 || r->node_width == 4, "node width 2 or 4");
   VRX_ARG(r->defer_steps >= 0, "defer_steps");
   VRX_ARG(!wide_of(r) || scene->num_entries == 0 || scene->wide,
-      "node width 4 needs 4-wide nodes for every BVH (vrx_bvh_widen, scene->wide)");
+      "node width 4 needs 4-wide nodes for every BVH (vrx_bvh_pack or vrx_bvh_widen, scene->wide)");
   uint32_t sd = pick_sd(r);
   uint32_t cap = ovf_cap_of(scene, sd, wide_of(r));
   size_t need = vrx_render_scratch_bytes(scene, r, f->width, f->height);

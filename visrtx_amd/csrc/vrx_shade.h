@@ -603,7 +603,7 @@ __device__ __forceinline__ void wave_count_add(uint64_t *ctrs, uint32_t c, uint3
 // reached 0.99 counts as fully blocked: which hits the reference visits before
 // it stops depends on its traversal order, so its value then lies anywhere in
 // [0.99, 1]; below 0.99 every hit is visited and the value is the same.
-template <int PT, bool TWO, bool WIDE>
+template <int PT, bool TWO, int WIDE>
 __device__ __forceinline__ float surface_atten(
     const vrx_scene &sc, v3 o, v3 d, float tmax, Stack &st, uint32_t &rays)
 {
@@ -616,7 +616,7 @@ __device__ __forceinline__ float surface_atten(
 
 // computeAO (gpu/computeAO.h:38-60): n cosine-weighted hemisphere rays from
 // the geometric-normal offset point, four PCG draws each.
-template <int PT, bool TWO, bool WIDE>
+template <int PT, bool TWO, int WIDE>
 __device__ float ao_factor(const vrx_scene &sc, const SurfHit &s, float dist, int n, Pcg &rs,
     Stack &st, uint32_t &rays)
 {
@@ -711,7 +711,7 @@ __device__ __forceinline__ LightSample sample_light(const vrx_light *L, v3 hp)
 // shadow ray from the shading point.  Matte surfaces spawn no bounce ray
 // (their nextRay is zero), so the bounce loop ends at once.  Returns the
 // colour and the material opacity.
-template <int PT, bool TWO, bool WIDE>
+template <int PT, bool TWO, int WIDE>
 __device__ float4 shade_direct(const vrx_scene &sc, const vrx_renderer &r, const SurfHit &s,
     int aos, Pcg &rs, Stack &st, uint32_t &rays, uint32_t &vsamples)
 {
@@ -786,7 +786,7 @@ __device__ __forceinline__ void defer_pixel(const LongRays &lr, uint32_t idx)
 // Each lane keeps its own closest hit by take() (so ties resolve as in one
 // walk) and the group takes the closest over its lanes.  A push that would
 // overflow the shared stack goes to the lanes' private stacks instead.
-template <int PT, bool WIDE>
+template <int PT, int WIDE>
 __device__ __forceinline__ bool trace_group(const vrx_scene &sc, v3 wo, v3 wd, float tmin,
     float tmax, bool cull, Stack &st, Hit &h, uint32_t *gs, uint32_t gcap)
 {
@@ -804,10 +804,11 @@ __device__ __forceinline__ bool trace_group(const vrx_scene &sc, v3 wo, v3 wd, f
   load_blas(sc, 0u, wo, wd, cull, false, b, o, d, root, n);
   if (n == 0)
     return false;
-  const v3 inv = mk(1.0f / d.x, 1.0f / d.y, 1.0f / d.z);
+  const v3 inv = walk_inv<WIDE>(d);
   WT wt;
   if (blas_type<PT>(b) == VRX_TRIANGLE)
     wt = wt_setup(d);
+  std::conditional_t<WIDE == 2, BoxGuard<false>, NoGuard> guard;
   const uint32_t lane = threadIdx.x & 63u, s = lane & 15u;
   const uint64_t gmask = 0xFFFFull << (lane & ~15u);
   const uint64_t below = (1ull << lane) - 1ull;
@@ -837,21 +838,28 @@ __device__ __forceinline__ bool trace_group(const vrx_scene &sc, v3 wo, v3 wd, f
     uint32_t nout = 0;
     if (has) {
       if (WIDE && !(node & kLeafBit)) {
-        const Node4 nd = gld_node4(b.wnodes, node);
-        const float lx[4] = {nd.lox.x, nd.lox.y, nd.lox.z, nd.lox.w};
-        const float ly[4] = {nd.loy.x, nd.loy.y, nd.loy.z, nd.loy.w};
-        const float lz[4] = {nd.loz.x, nd.loz.y, nd.loz.z, nd.loz.w};
-        const float hx[4] = {nd.hix.x, nd.hix.y, nd.hix.z, nd.hix.w};
-        const float hy[4] = {nd.hiy.x, nd.hiy.y, nd.hiy.z, nd.hiy.w};
-        const float hz[4] = {nd.hiz.x, nd.hiz.y, nd.hiz.z, nd.hiz.w};
-        uint32_t l[4] = {nd.link.x, nd.link.y, nd.link.z, nd.link.w};
         float t[4];
+        uint32_t l[4];
+        if constexpr (WIDE == 2) {
+          const Node4p nd = gld_node4p((const Node4p *)b.wnodes, node);
+          l[0] = nd.link.x; l[1] = nd.link.y; l[2] = nd.link.z; l[3] = nd.link.w;
+          slab4p(nd, o, inv, tmin, tb, t);
+        } else {
+          const Node4 nd = gld_node4((const Node4 *)b.wnodes, node);
+          const float lx[4] = {nd.lox.x, nd.lox.y, nd.lox.z, nd.lox.w};
+          const float ly[4] = {nd.loy.x, nd.loy.y, nd.loy.z, nd.loy.w};
+          const float lz[4] = {nd.loz.x, nd.loz.y, nd.loz.z, nd.loz.w};
+          const float hx[4] = {nd.hix.x, nd.hix.y, nd.hix.z, nd.hix.w};
+          const float hy[4] = {nd.hiy.x, nd.hiy.y, nd.hiy.z, nd.hiy.w};
+          const float hz[4] = {nd.hiz.x, nd.hiz.y, nd.hiz.z, nd.hiz.w};
+          l[0] = nd.link.x; l[1] = nd.link.y; l[2] = nd.link.z; l[3] = nd.link.w;
 #pragma unroll
-        for (int c = 0; c < 4; c++) {
-          float tn;
-          const bool hit = (uint32_t)c < nd.meta.x
-              && slab(lx[c], ly[c], lz[c], hx[c], hy[c], hz[c], o, inv, tmin, tb, tn);
-          t[c] = hit ? tn : INFINITY;
+          for (int c = 0; c < 4; c++) {
+            float tn;
+            const bool hit = (uint32_t)c < nd.meta.x
+                && slab(lx[c], ly[c], lz[c], hx[c], hy[c], hz[c], o, inv, tmin, tb, tn);
+            t[c] = hit ? tn : INFINITY;
+          }
         }
         cswap(t[0], l[0], t[1], l[1]);
         cswap(t[2], l[2], t[3], l[3]);
@@ -881,7 +889,8 @@ __device__ __forceinline__ bool trace_group(const vrx_scene &sc, v3 wo, v3 wd, f
         }
       } else {
         float tcur = h.t;
-        (void)test_leaf<PT, false>(b, node & ~kLeafBit, o, d, wt, tmin, tcur, h);
+        if (WIDE != 2 || node != kPackEmpty)
+          (void)test_leaf<PT, false>(b, node & ~kLeafBit, o, d, wt, tmin, tcur, h, guard);
         has = false;
       }
     }
@@ -946,7 +955,7 @@ __device__ __forceinline__ bool trace_group(const vrx_scene &sc, v3 wo, v3 wd, f
 // over lr.budget iterations queue their pixel and write nothing; 2 = the
 // pixel's walks are shared by its 16-lane group (trace_group), and the
 // group's first lane writes it.
-template <int PT, bool TWO, int KIND, bool WIDE = false, int LONG = 0>
+template <int PT, bool TWO, int KIND, int WIDE = 0, int LONG = 0>
 __device__ __forceinline__ void render_pixel(const vrx_scene &sc, const vrx_camera &cam,
     const vrx_renderer &r, const vrx_frame &f, uint32_t px, uint32_t py, size_t idx, Stack &st,
     uint32_t &rays, uint32_t &vsamples, const LongRays *lr = nullptr)

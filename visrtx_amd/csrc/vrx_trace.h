@@ -15,6 +15,8 @@
 // traversal order, so it is the same hit the CPU brute force finds.
 #pragma once
 
+#include <type_traits>
+
 #include "vrx_lbvh.h"
 #include "vrx_math.h"
 
@@ -240,12 +242,13 @@ struct Hit {
 
 struct BlasCtx {
   const Node *nodes;
-  const Node4 *wnodes; // 4-wide nodes (traversal of width 4 only)
+  const void *wnodes;  // 4-wide nodes (Node4 or Node4p; traversal of width 4 only)
   const float4 *leaves;
   const uint32_t *ids;
   int type;
   bool cull;
   bool caps;
+  bool boxed;    // the BVH has inner nodes: a leaf is reached through its box
   uint32_t entry;
   float opacity; // surface opacity (any-hit rays only)
 };
@@ -258,7 +261,7 @@ __device__ __forceinline__ void load_blas(
   const uint32_t gi = gld(&Ep->geom);
   const vrx_geom *G = sc.d_geoms + gi;
   b.nodes = (const Node *)gld(&G->bvh.d_nodes);
-  b.wnodes = (const Node4 *)gld(&G->bvh.d_wide);
+  b.wnodes = gld(&G->bvh.d_wide);
   b.leaves = (const float4 *)gld(&G->bvh.d_leaves);
   b.ids = gld(&G->bvh.d_leaf_ids);
   b.type = gld(&G->type);
@@ -268,6 +271,7 @@ __device__ __forceinline__ void load_blas(
   b.opacity = any ? gld(&G->opacity) : 1.0f;
   n = gld(&G->n);
   root = n == 1 ? kLeafBit : 0u;
+  b.boxed = n > 1;
   if (gld(&Ep->identity)) {
     o = wo;
     d = wd;
@@ -412,16 +416,60 @@ __device__ __forceinline__ bool any_hit(const BlasCtx &b, Hit &h)
   return !(h.a0 < 0.99f);
 }
 
+// Full-precision nodes: a leaf is reached only through its exact box.
+struct NoGuard {
+  static constexpr bool on = false;
+};
+
+// Packed nodes enclose more than the exact boxes, so a walk can reach a leaf
+// that the exact boxes cull (a grazing ray whose primitive test reports a hit
+// by rounding).  A reported hit therefore also has to pass the slab test of
+// its leaf's exact box and, under instances, of its entry's box.  Those two
+// decide for all boxes above them, which contain them (the slab distances
+// are monotonic in the planes), so the accepted hits are those of a walk over
+// exact boxes.  Only reported hits pay for it, about one per ray.
+template <bool TWO>
+struct BoxGuard {
+  static constexpr bool on = true;
+  const float *entry_box; // 6 floats per entry (TWO)
+  v3 wo, wd;              // the ray in world space (TWO)
+
+  template <int T>
+  __device__ __forceinline__ bool pass(
+      const BlasCtx &b, const float4 *rec, v3 o, v3 d, float tmin, float tmax) const
+  {
+    float tn;
+    if (b.boxed) {
+      v3 lo, hi;
+      record_box<T>(rec, lo, hi);
+      const v3 inv = mk(1.0f / d.x, 1.0f / d.y, 1.0f / d.z);
+      if (!slab(lo.x, lo.y, lo.z, hi.x, hi.y, hi.z, o, inv, tmin, tmax, tn))
+        return false;
+    }
+    if constexpr (TWO) {
+      const float *e = entry_box + 6 * (size_t)b.entry;
+      const v3 inv = mk(1.0f / wd.x, 1.0f / wd.y, 1.0f / wd.z);
+      return slab(gld(e, 0), gld(e, 1), gld(e, 2), gld(e, 3), gld(e, 4), gld(e, 5), wo, inv, tmin,
+          tmax, tn);
+    }
+    return true;
+  }
+};
+
 // Test leaf k of the current BLAS.  Returns true for an any-hit termination.
-template <int PT, bool ANY>
-__device__ __forceinline__ bool test_leaf(
-    const BlasCtx &b, uint32_t k, v3 o, v3 d, const WT &wt, float tmin, float &tmax, Hit &h)
+template <int PT, bool ANY, class Guard>
+__device__ __forceinline__ bool test_leaf(const BlasCtx &b, uint32_t k, v3 o, v3 d, const WT &wt,
+    float tmin, float &tmax, Hit &h, const Guard &guard)
 {
   const int type = blas_type<PT>(b);
   if (type == VRX_SPHERE) {
     float4 L = gld(b.leaves, k);
     float t;
     if (isect_sphere(o, d, mk(L.x, L.y, L.z), L.w, t) && t >= tmin && t <= tmax) {
+      if constexpr (Guard::on) {
+        if (!guard.template pass<VRX_SPHERE>(b, &L, o, d, tmin, tmax))
+          return false;
+      }
       if (ANY)
         return any_hit(b, h);
       uint32_t prim = gld(b.ids, k);
@@ -444,6 +492,11 @@ __device__ __forceinline__ bool test_leaf(
         if (!(dot(ng, d) < 0.0f))
           return false;
       }
+      if constexpr (Guard::on) {
+        const float4 rec[3] = {A, B, C};
+        if (!guard.template pass<VRX_TRIANGLE>(b, rec, o, d, tmin, tmax))
+          return false;
+      }
       if (ANY)
         return any_hit(b, h);
       uint32_t prim = gld(b.ids, k);
@@ -464,6 +517,11 @@ __device__ __forceinline__ bool test_leaf(
     v3 ns[3];
     int vm = isect_cylinder(o, d, mk(P0.x, P0.y, P0.z), mk(P1.x, P1.y, P1.z), P0.w,
         b.caps, ts, ns);
+    if constexpr (Guard::on) {
+      const float4 rec[2] = {P0, P1};
+      if (vm && !guard.template pass<VRX_CYLINDER>(b, rec, o, d, tmin, tmax))
+        return false;
+    }
 #pragma unroll
     for (int q = 0; q < 3; q++) {
       if (!(vm & (1 << q)))
@@ -495,6 +553,11 @@ __device__ __forceinline__ bool test_leaf(
     v3 nn;
     if (isect_round_cone(o, d, mk(P0.x, P0.y, P0.z), mk(P1.x, P1.y, P1.z), P0.w, P1.w, t, nn)
         && t >= tmin && t <= tmax) {
+      if constexpr (Guard::on) {
+        const float4 rec[2] = {P0, P1};
+        if (!guard.template pass<VRX_CURVE>(b, rec, o, d, tmin, tmax))
+          return false;
+      }
       if (ANY)
         return any_hit(b, h);
       uint32_t prim = gld(b.ids, k);
@@ -515,6 +578,11 @@ __device__ __forceinline__ bool test_leaf(
     float ts[2];
     v3 ns[2];
     int vm = isect_cone(o, d, mk(P0.x, P0.y, P0.z), mk(P1.x, P1.y, P1.z), P0.w, P1.w, ts, ns);
+    if constexpr (Guard::on) {
+      const float4 rec[2] = {P0, P1};
+      if (vm && !guard.template pass<VRX_CONE>(b, rec, o, d, tmin, tmax))
+        return false;
+    }
 #pragma unroll
     for (int q = 0; q < 2; q++) {
       if (!(vm & (1 << q)))
@@ -596,9 +664,90 @@ __device__ __forceinline__ bool visit4(const Node4 &nd, v3 o, v3 inv, float tmin
   return true;
 }
 
+// Reciprocal directions for the packed nodes' plane distances: a zero
+// direction component gives 2^100 instead of infinity, so that a plane
+// through the grid origin does not become 0 * infinity.
+__device__ __forceinline__ v3 pack_inv(v3 d)
+{
+  constexpr float big = 0x1p100f;
+  return mk(fminf(fmaxf(1.0f / d.x, -big), big), fminf(fmaxf(1.0f / d.y, -big), big),
+      fminf(fmaxf(1.0f / d.z, -big), big));
+}
+
+// slack of the packed slab test, on the far side alone: the 2^-18 of slab()
+// on either side (2^-17 between them), and as much again for the rounding of
+// the plane distances where the ray origin is far outside the grid (there
+// within 2^-22 of the distance; nearer, kPackMargin covers it)
+constexpr float kPackHi = 1.0f + 0x1p-16f;
+
+__device__ __forceinline__ float pack_byte(uint32_t w, int c)
+{
+  return (float)((w >> (8 * c)) & 255u); // v_cvt_f32_ubyte
+}
+
+// Entry distance of the children of a packed node (infinity: missed).  The
+// distance of plane q is q * (scale * inv) + (origin - o) * inv, one FMA; the
+// near and far planes of all four children are picked by the ray's sign, one
+// word per axis.
+__device__ __forceinline__ void slab4p(const Node4p &nd, v3 o, v3 inv, float tmin, float tmax,
+    float t[4])
+{
+  const float ax = nd.sx * inv.x, ay = nd.sy * inv.y, az = nd.sz * inv.z;
+  const float bx = (nd.ox - o.x) * inv.x, by = (nd.oy - o.y) * inv.y, bz = (nd.oz - o.z) * inv.z;
+  const bool px = inv.x >= 0.0f, py = inv.y >= 0.0f, pz = inv.z >= 0.0f;
+  const uint32_t nx = px ? nd.lox : nd.hix, fx = px ? nd.hix : nd.lox;
+  const uint32_t ny = py ? nd.loy : nd.hiy, fy = py ? nd.hiy : nd.loy;
+  const uint32_t nz = pz ? nd.loz : nd.hiz, fz = pz ? nd.hiz : nd.loz;
+  const float cap = tmax * kPackHi;
+#pragma unroll
+  for (int c = 0; c < 4; c++) {
+    const float tn = fmaxf(fmaxf(fmaxf(__builtin_fmaf(pack_byte(nx, c), ax, bx),
+                                     __builtin_fmaf(pack_byte(ny, c), ay, by)),
+                               __builtin_fmaf(pack_byte(nz, c), az, bz)), tmin);
+    const float tf = fminf(fminf(__builtin_fmaf(pack_byte(fx, c), ax, bx),
+                               __builtin_fmaf(pack_byte(fy, c), ay, by)),
+        __builtin_fmaf(pack_byte(fz, c), az, bz));
+    t[c] = tn <= fminf(tf * kPackHi, cap) ? tn : INFINITY;
+  }
+}
+
+// visit4() on a packed node
+__device__ __forceinline__ bool visit4p(const Node4p &nd, v3 o, v3 inv, float tmin, float tmax,
+    Stack &st, uint32_t &node)
+{
+  uint32_t l[4] = {nd.link.x, nd.link.y, nd.link.z, nd.link.w};
+  float t[4];
+  slab4p(nd, o, inv, tmin, tmax, t);
+  cswap(t[0], l[0], t[1], l[1]);
+  cswap(t[2], l[2], t[3], l[3]);
+  cswap(t[0], l[0], t[2], l[2]);
+  cswap(t[1], l[1], t[3], l[3]);
+  cswap(t[1], l[1], t[2], l[2]);
+  if (!(t[0] < INFINITY))
+    return false;
+  if (t[3] < INFINITY)
+    st.push(l[3]);
+  if (t[2] < INFINITY)
+    st.push(l[2]);
+  if (t[1] < INFINITY)
+    st.push(l[1]);
+  node = l[0];
+  return true;
+}
+
+template <int WIDE>
+__device__ __forceinline__ v3 walk_inv(v3 d)
+{
+  if constexpr (WIDE == 2)
+    return pack_inv(d);
+  else
+    return mk(1.0f / d.x, 1.0f / d.y, 1.0f / d.z);
+}
+
+// WIDE: 0 BVH2 nodes, 1 the 128-byte 4-wide nodes, 2 the packed ones.
 // BUDGET: the walk gives up after `budget` loop iterations and sets
 // *deferred (the caller finishes that ray another way); h is then partial.
-template <int PT, bool TWO_LEVEL, bool ANY, bool WIDE = false, bool BUDGET = false>
+template <int PT, bool TWO_LEVEL, bool ANY, int WIDE = 0, bool BUDGET = false>
 __device__ bool trace(const vrx_scene &sc, v3 wo, v3 wd, float tmin, float tmax, bool cull_all,
     Stack &st, Hit &h, uint32_t budget = 0, bool *deferred = nullptr)
 {
@@ -610,17 +759,17 @@ __device__ bool trace(const vrx_scene &sc, v3 wo, v3 wd, float tmin, float tmax,
   if (sc.num_entries == 0)
     return false;
   st.cnt = 0;
-  const v3 winv = mk(1.0f / wd.x, 1.0f / wd.y, 1.0f / wd.z);
+  const v3 winv = walk_inv<WIDE>(wd);
   v3 o = wo, d = wd, inv = winv;
   WT wt;
   BlasCtx b;
   bool in_blas;
   uint32_t node;
   const Node *nodes;
-  const Node4 *wnodes = nullptr;
+  const void *wnodes = nullptr;
   const uint32_t *tlas_ids = sc.tlas.d_leaf_ids;
   const Node *tlas_nodes = (const Node *)sc.tlas.d_nodes;
-  const Node4 *tlas_wnodes = (const Node4 *)sc.tlas.d_wide;
+  const void *tlas_wnodes = sc.tlas.d_wide;
   if (TWO_LEVEL) {
     in_blas = false;
     nodes = tlas_nodes;
@@ -631,13 +780,22 @@ __device__ bool trace(const vrx_scene &sc, v3 wo, v3 wd, float tmin, float tmax,
     load_blas(sc, 0u, wo, wd, cull_all, ANY, b, o, d, root, n);
     if (n == 0)
       return false;
-    inv = mk(1.0f / d.x, 1.0f / d.y, 1.0f / d.z);
+    inv = walk_inv<WIDE>(d);
     if (blas_type<PT>(b) == VRX_TRIANGLE)
       wt = wt_setup(d);
     in_blas = true;
     nodes = b.nodes;
     wnodes = b.wnodes;
     node = root;
+  }
+  using Guard = std::conditional_t<WIDE == 2, BoxGuard<TWO_LEVEL>, NoGuard>;
+  Guard guard;
+  if constexpr (WIDE == 2) {
+    // the packed instance nodes are followed by the entries' exact boxes
+    guard.entry_box = TWO_LEVEL
+        ? (const float *)((const Node4p *)sc.tlas.d_wide + (sc.num_entries - 1)) : nullptr;
+    guard.wo = wo;
+    guard.wd = wd;
   }
   [[maybe_unused]] uint32_t iters = 0;
   for (;;) {
@@ -648,8 +806,13 @@ __device__ bool trace(const vrx_scene &sc, v3 wo, v3 wd, float tmin, float tmax,
       }
     }
     bool do_pop = true;
-    if (WIDE && !(node & kLeafBit)) {
-      const Node4 nd = gld_node4(wnodes, node);
+    if (WIDE == 2 && !(node & kLeafBit)) {
+      const Node4p nd = gld_node4p((const Node4p *)wnodes, node);
+      do_pop = !visit4p(nd, o, inv, tmin, h.t, st, node);
+    } else if (WIDE == 2 && node == kPackEmpty) {
+      // an unused slot, "hit" where rounding swallows the whole grid
+    } else if (WIDE == 1 && !(node & kLeafBit)) {
+      const Node4 nd = gld_node4((const Node4 *)wnodes, node);
       do_pop = !visit4(nd, o, inv, tmin, h.t, st, node);
     } else if (!(node & kLeafBit)) {
       const Node nd = gld_node(nodes, node);
@@ -674,7 +837,7 @@ __device__ bool trace(const vrx_scene &sc, v3 wo, v3 wd, float tmin, float tmax,
       }
     } else if (in_blas) {
       float tcur = h.t;
-      if (test_leaf<PT, ANY>(b, node & ~kLeafBit, o, d, wt, tmin, tcur, h))
+      if (test_leaf<PT, ANY>(b, node & ~kLeafBit, o, d, wt, tmin, tcur, h, guard))
         return true;
     } else {
       // instance leaf: enter the entry's BLAS in object space
@@ -682,7 +845,7 @@ __device__ bool trace(const vrx_scene &sc, v3 wo, v3 wd, float tmin, float tmax,
       uint32_t n, root;
       load_blas(sc, e, wo, wd, cull_all, ANY, b, o, d, root, n);
       if (n != 0) {
-        inv = mk(1.0f / d.x, 1.0f / d.y, 1.0f / d.z);
+        inv = walk_inv<WIDE>(d);
         if (blas_type<PT>(b) == VRX_TRIANGLE)
           wt = wt_setup(d);
         st.push(kMarker);
