@@ -82,6 +82,49 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(6, 8))) 
   render_tile<PT, TWO, KIND, WIDE>(sc, cam, r, f, sd, ovf_cap, scratch);
 }
 
+// The sampled renderers on packed nodes, a wave per 8x8 tile (render_wave()),
+// over a resident grid: each wave owns a ray queue in memory and takes the
+// next tile from a counter (header word 2 of the scratch).
+template <int PT, bool TWO, int KIND>
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(5, 8))) void
+k_render_sampled(vrx_scene sc, vrx_camera cam, vrx_renderer r, vrx_frame f, uint32_t sd,
+    uint32_t ovf_cap, uint32_t *scratch, float *queues, uint32_t tiles_x, uint32_t tiles)
+{
+  extern __shared__ uint32_t s_stack[];
+  __shared__ uint16_t s_codes[kBlock / 64][kQueueSlots * 64];
+  const uint32_t tid = threadIdx.x, wave = tid >> 6, lane = tid & 63u;
+  Stack st;
+  st.lds = s_stack + tid;
+  st.stride = kBlock;
+  st.sd = sd;
+  st.sd_mask = sd - 1;
+  st.ovf = scratch + 64 + blockIdx.x * kBlock + tid;
+  st.ovf_stride = gridDim.x * kBlock;
+  st.ovf_cap = ovf_cap;
+  st.err = scratch;
+  st.cnt = 0;
+  RayQueue q;
+  q.mem = queues + (size_t)(blockIdx.x * (kBlock / 64) + wave) * kQueueFloats;
+  q.codes = s_codes[wave];
+  q.n = 0;
+  uint32_t rays = 0;
+  for (;;) {
+    uint32_t t = 0;
+    if (lane == 0)
+      t = atomicAdd(scratch + 2, 1u);
+    t = (uint32_t)__builtin_amdgcn_readfirstlane((int)t);
+    if (t >= tiles)
+      break;
+    const uint32_t ty = t / tiles_x, tx = t - ty * tiles_x;
+    const uint32_t px = tx * 8 + (lane & 7u), py = ty * 8 + (lane >> 3);
+    const bool inside = px < f.width && py < f.height;
+    render_wave<PT, TWO, KIND>(sc, cam, r, f, px, py, inside, (size_t)px + (size_t)py * f.width, st,
+        q, rays);
+  }
+  if (f.d_counters)
+    wave_count_add(f.d_counters, 0, rays);
+}
+
 // The one-level primitive raycast with a step budget: walks longer than
 // lr.budget loop iterations queue their pixel for k_render_long.
 template <int PT, int WIDE>
@@ -653,6 +696,37 @@ static size_t long_queue_offset(uint32_t width, uint32_t height, uint32_t cap)
   return 256 + tiles * kBlock * (size_t)cap * 4;
 }
 
+// Byte offset of the ray queues in the frame scratch (after the stack-spill
+// area) and their bytes: one queue per wave of the largest resident grid.
+static uint32_t sampled_max_blocks(uint32_t width, uint32_t height)
+{
+  const uint64_t tiles = (uint64_t)((width + kTile - 1) / kTile) * ((height + kTile - 1) / kTile);
+  return (uint32_t)std::min<uint64_t>(tiles, (uint64_t)device_cus() * 8);
+}
+
+static size_t sampled_queue_bytes(uint32_t width, uint32_t height)
+{
+  return (size_t)sampled_max_blocks(width, height) * (kBlock / 64) * kQueueFloats * 4;
+}
+
+// Scenes and renderers k_render_sampled takes: AO and directLight on packed
+// nodes, one primitive type, no volumes.
+static bool sampled_applies(const vrx_scene *sc, const vrx_renderer *r)
+{
+  return r && wide_of(r) && sc->wide_format == VRX_WIDE_PACKED && sc->num_volumes == 0
+      && sc->single_type >= VRX_TRIANGLE && sc->single_type <= VRX_CYLINDER
+      && (r->kind == VRX_RENDER_AO || r->kind == VRX_RENDER_DIRECT);
+}
+
+// scratch of every launch: header, stack spill, the long-ray queue
+static size_t base_scratch_bytes(const vrx_scene *scene, const vrx_renderer *r, uint32_t width,
+    uint32_t height)
+{
+  const uint32_t cap = ovf_cap_of(scene, pick_sd(r), wide_of(r));
+  const size_t queue = r && r->defer_steps > 0 ? (size_t)width * height * 4 : 0;
+  return (long_queue_offset(width, height, cap) + queue + 255) & ~size_t(255);
+}
+
 template <int PT, bool TWO, int KIND, int WIDE>
 static void launch_one(const vrx_scene &sc, const vrx_camera &cam, const vrx_renderer &r,
     const vrx_frame &f, uint32_t sd, uint32_t cap, hipStream_t s)
@@ -687,6 +761,25 @@ static void launch_one(const vrx_scene &sc, const vrx_camera &cam, const vrx_ren
       const uint32_t blocks = std::min((uint32_t)(per_cu * device_cus()), grid.x * grid.y);
       hipLaunchKernelGGL((k_render_long<PT, WIDE>), dim3(blocks), dim3(kBlock), lds2, s, sc, cam,
           r, f, sd, cap, (uint32_t *)f.d_scratch, lr);
+      return;
+    }
+  }
+  if constexpr (PT >= 0 && KIND != VRX_RENDER_RAYCAST && WIDE == 2) {
+    // a caller whose scratch was sized without the queues keeps the per-pixel kernel
+    const size_t off = base_scratch_bytes(&sc, &r, f.width, f.height);
+    if (f.scratch_bytes >= off + sampled_queue_bytes(f.width, f.height)) {
+      const void *kern = (const void *)&k_render_sampled<PT, TWO, KIND>;
+      int per_cu = 0;
+      if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kern, kBlock, lds) != hipSuccess
+          || per_cu < 1)
+        per_cu = 1;
+      const uint32_t tx = (f.width + 7) / 8, ty = (f.height + 7) / 8;
+      const uint32_t blocks = std::min(std::min((uint32_t)(per_cu * device_cus()),
+          sampled_max_blocks(f.width, f.height)), (tx * ty + 3) / 4);
+      (void)vrx_fill_u32((uint32_t *)f.d_scratch + 2, 0u, 1, (vrx_stream)s);
+      hipLaunchKernelGGL((k_render_sampled<PT, TWO, KIND>), dim3(blocks), dim3(kBlock), lds, s, sc,
+          cam, r, f, sd, cap, (uint32_t *)f.d_scratch, (float *)((char *)f.d_scratch + off), tx,
+          tx * ty);
       return;
     }
   }
@@ -744,10 +837,8 @@ size_t vrx_render_scratch_bytes(const vrx_scene *scene, const vrx_renderer *r, u
 {
   if (!scene)
     return 0;
-  uint32_t sd = pick_sd(r);
-  uint32_t cap = ovf_cap_of(scene, sd, wide_of(r));
-  const size_t queue = r && r->defer_steps > 0 ? (size_t)width * height * 4 : 0;
-  return long_queue_offset(width, height, cap) + queue;
+  return base_scratch_bytes(scene, r, width, height)
+      + (sampled_applies(scene, r) ? sampled_queue_bytes(width, height) : 0);
 }
 
 int vrx_frame_clear(const vrx_frame *f, vrx_stream s)
@@ -779,7 +870,7 @@ int vrx_render(const vrx_scene *scene, const vrx_camera *cam, const vrx_renderer
       "node width 4 needs 4-wide nodes for every BVH (vrx_bvh_pack or vrx_bvh_widen, scene->wide)");
   uint32_t sd = pick_sd(r);
   uint32_t cap = ovf_cap_of(scene, sd, wide_of(r));
-  size_t need = vrx_render_scratch_bytes(scene, r, f->width, f->height);
+  size_t need = base_scratch_bytes(scene, r, f->width, f->height);
   if (!f->d_scratch || f->scratch_bytes < need) {
     set_error("render scratch too small: %zu < %zu", f->scratch_bytes, need);
     return VRX_ERR_ARG;

@@ -945,6 +945,405 @@ __device__ __forceinline__ bool trace_group(const vrx_scene &sc, v3 wo, v3 wd, f
 }
 
 // --------------------------------------------------------------------------
+// sampled pixels a wave at a time: secondary rays through a queue
+// --------------------------------------------------------------------------
+// The AO / directLight program of render_pixel() for a wave of 64 pixels in
+// step.  In render_pixel() a wave's secondary rays run one per lane and wait
+// for the longest: only a third of the lanes work in their node visits
+// (pixels that missed have none, the rest end at different times).  Here the
+// lanes write their AO and shadow rays to the wave's queue, of several samples
+// where their pixels are opaque, and the 64 lanes take rays off it as they
+// finish.  The results are then summed per pixel in render_pixel()'s order,
+// and the random draws are the same, so the pixels are the same.
+// Measured against render_pixel() on the same nodes: AO 16 spp on 10M spheres
+// 11.1 -> 10.8 ms with 1 AO ray per hit (closest walks are half of the steps
+// there), 4 spp with 2 lights and 1 AO ray on 1M spheres 3.84 -> 3.10 ms;
+// 3 slots instead of 6 are 4 % slower, 12 as fast; workgroup-wide tiles 6 %
+// slower than a tile per wave (its waves wait for one another).
+constexpr int kQueueSlots = 6;    // rays per pixel and round
+constexpr int kQueueWords = 12;   // origin, direction, weight (3), tmax, result, unused
+constexpr int kSampleWords = 4;   // surface colour and opacity
+constexpr uint32_t kQueueFloats = (kQueueSlots * (kQueueWords + kSampleWords)) * 64; // per wave
+
+struct RayQueue {
+  float *mem;       // this wave's kQueueFloats words, word-major ([word][lane])
+  uint16_t *codes;  // LDS: slot * 64 + lane of the queued rays
+  uint32_t n;       // queued rays
+};
+
+__device__ __forceinline__ float *queue_ray(const RayQueue &q, uint32_t slot, uint32_t word)
+{
+  return q.mem + (slot * kQueueWords + word) * 64;
+}
+
+__device__ __forceinline__ float *queue_sample(const RayQueue &q, uint32_t s, uint32_t word)
+{
+  return q.mem + (kQueueSlots * kQueueWords + s * kSampleWords + word) * 64;
+}
+
+// the wave's memory and LDS operations before this are done and visible to its lanes
+__device__ __forceinline__ void wave_mem_sync()
+{
+  __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "workgroup");
+  __builtin_amdgcn_wave_barrier();
+}
+
+// queue this lane's ray in `slot` (valid lanes only; called by the whole wave)
+__device__ __forceinline__ void queue_push(RayQueue &q, uint32_t slot, uint32_t lane, bool valid,
+    v3 o, v3 d, v3 w, float tmax)
+{
+  const uint64_t m = __ballot(valid);
+  if (valid) {
+    const uint32_t rank = __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32),
+        __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
+    q.codes[q.n + rank] = (uint16_t)(slot * 64 + lane);
+    gst(queue_ray(q, slot, 0), lane, o.x);
+    gst(queue_ray(q, slot, 1), lane, o.y);
+    gst(queue_ray(q, slot, 2), lane, o.z);
+    gst(queue_ray(q, slot, 3), lane, d.x);
+    gst(queue_ray(q, slot, 4), lane, d.y);
+    gst(queue_ray(q, slot, 5), lane, d.z);
+    gst(queue_ray(q, slot, 6), lane, w.x);
+    gst(queue_ray(q, slot, 7), lane, w.y);
+    gst(queue_ray(q, slot, 8), lane, w.z);
+    gst(queue_ray(q, slot, 9), lane, tmax);
+  }
+  q.n += (uint32_t)__popcll(m);
+}
+
+// Trace the queued rays (the whole wave): lanes without a ray take the next
+// ones once a quarter of the wave waits for one.
+template <int PT, bool TWO>
+__device__ __forceinline__ void queue_drain(const vrx_scene &sc, RayQueue &q, uint32_t lane,
+    Stack &st)
+{
+  wave_mem_sync();
+  Walk<PT, TWO, true> w;
+  const bool scene = w.attach(sc, false);
+  uint32_t head = 0, slot = 0, owner = 0;
+  bool have = false;
+  for (;;) {
+    const uint64_t idle = __ballot(!have);
+    if (head < q.n) {
+      if (!have) {
+        const uint32_t i = head + __builtin_amdgcn_mbcnt_hi((uint32_t)(idle >> 32),
+            __builtin_amdgcn_mbcnt_lo((uint32_t)idle, 0u));
+        if (i < q.n) {
+          const uint32_t code = q.codes[i];
+          slot = code >> 6;
+          owner = code & 63u;
+          const v3 o = mk(gld(queue_ray(q, slot, 0), owner), gld(queue_ray(q, slot, 1), owner),
+              gld(queue_ray(q, slot, 2), owner));
+          const v3 d = mk(gld(queue_ray(q, slot, 3), owner), gld(queue_ray(q, slot, 4), owner),
+              gld(queue_ray(q, slot, 5), owner));
+          const float tmax = gld(queue_ray(q, slot, 9), owner);
+          if (scene) {
+            w.begin(sc, o, d, 0.0f, tmax, st);
+            have = true;
+          } else {
+            gst(queue_ray(q, slot, 10), owner, 0.0f);
+          }
+        }
+      }
+      head += (uint32_t)__popcll(idle);
+    } else if (idle == ~0ull) {
+      break;
+    }
+    // steps until a quarter of the wave waits (or, with the queue empty, all of it)
+    const int limit = head < q.n ? 16 : 64;
+    do {
+      if (have && w.step(sc, false, st)) {
+        // an opacity that reached 0.99 counts as blocked, as in surface_atten()
+        gst(queue_ray(q, slot, 10), owner, !(w.h.a0 < 0.99f) ? 1.0f : w.h.a0);
+        have = false;
+      }
+    } while ((int)__popcll(__ballot(!have)) < limit);
+  }
+  q.n = 0;
+  wave_mem_sync();
+}
+
+// the sum of the secondary rays of one shading point
+struct SecondarySum {
+  float weights, hits;
+  v3 contrib;
+};
+
+// add the results of secondary rays q0 .. q1-1 (in `slot` on) of a pixel
+template <int KIND>
+__device__ __forceinline__ void add_secondary(const vrx_scene &sc, const RayQueue &q, uint32_t slot,
+    uint32_t lane, int q0, int q1, int aos, uint32_t valid, SecondarySum &s)
+{
+  for (int k = q0; k < q1; k++, slot++) {
+    const bool v = (valid >> slot) & 1u;
+    const float occ = v ? gld(queue_ray(q, slot, 10), lane) : 0.0f;
+    if (k < aos) {
+      // a ray of weight 0 is not traced
+      const float wgt = v ? gld(queue_ray(q, slot, 6), lane) : 0.0f;
+      s.weights += wgt;
+      if (v)
+        s.hits += wgt * occ;
+    } else if (KIND == VRX_RENDER_DIRECT && v) {
+      const v3 c = mk(gld(queue_ray(q, slot, 6), lane), gld(queue_ray(q, slot, 7), lane),
+          gld(queue_ray(q, slot, 8), lane));
+      const float so = 1.0f - occ;
+      s.contrib = add(s.contrib, mulf(c, so * 1.0f));
+    }
+  }
+}
+
+// the layer's colour over what lies before it (outc, outo), as render_pixel() does
+template <int KIND>
+__device__ __forceinline__ void shade_layer(const vrx_renderer &r, const SecondarySum &s, int aos,
+    v3 scol, float sop, v3 &outc, float &outo)
+{
+  const float aof = aos > 0 ? (s.weights > 0.0f ? 1.0f - s.hits / s.weights : 0.0f) : 1.0f;
+  v3 color = mk(0.0f, 0.0f, 0.0f);
+  float opacity = 0.0f;
+  if (KIND == VRX_RENDER_DIRECT) {
+    const v3 sr = mulf(s.contrib, aof);
+    if (!(sr.x != sr.x || sr.y != sr.y || sr.z != sr.z)) {
+      color = sr;
+      opacity = sop;
+    }
+    const float w = 1.0f - opacity;
+    color = mk(color.x + sr.x * w, color.y + sr.y * w, color.z + sr.z * w);
+    opacity = opacity + sop * (1.0f - opacity);
+  } else {
+    const float scl = aof * r.ambient_radiance;
+    const v3 bl = mulv(scol, fmul(scl, ld3(r.ambient_color)));
+    const float w = 1.0f - opacity;
+    color = mk(color.x + bl.x * w, color.y + bl.y * w, color.z + bl.z * w);
+    opacity = opacity + sop * (1.0f - opacity);
+  }
+  color = mulf(color, opacity);
+  const float wo = 1.0f - outo;
+  outc = mk(outc.x + color.x * wo, outc.y + color.y * wo, outc.z + color.z * wo);
+  outo = outo + opacity * (1.0f - outo);
+}
+
+__device__ __forceinline__ void shade_miss(const vrx_renderer &r, v3 &outc, float &outo)
+{
+  v3 color = mulf(mk(0.0f, 0.0f, 0.0f), 0.0f);
+  float opacity = 0.0f;
+  const float w = 1.0f - opacity;
+  color = mk(color.x + r.background[0] * w, color.y + r.background[1] * w,
+      color.z + r.background[2] * w);
+  opacity = opacity + r.background[3] * (1.0f - opacity);
+  const float wo = 1.0f - outo;
+  outc = mk(outc.x + color.x * wo, outc.y + color.y * wo, outc.z + color.z * wo);
+  outo = outo + opacity * (1.0f - outo);
+}
+
+__device__ __forceinline__ void add_sample(v3 outc, float outo, float4 &accum)
+{
+  // accumResults (gpu_util.h:393-443)
+  const float ts = 1.0f + fmaxf(0.0f, cmax3(outc));
+  accum.x = accum.x + outc.x / ts;
+  accum.y = accum.y + outc.y / ts;
+  accum.z = accum.z + outc.z / ts;
+  accum.w = accum.w + outo;
+}
+
+// All pixels of a wave (px, py; `inside`: in the frame), packed nodes, scenes
+// of one primitive type without volumes.
+template <int PT, bool TWO, int KIND>
+__device__ __forceinline__ void render_wave(const vrx_scene &sc, const vrx_camera &cam,
+    const vrx_renderer &r, const vrx_frame &f, uint32_t px, uint32_t py, bool inside, size_t idx,
+    Stack &st, RayQueue &q, uint32_t &rays)
+{
+  static_assert(PT >= 0 && (KIND == VRX_RENDER_AO || KIND == VRX_RENDER_DIRECT),
+      "sampled renderers on scenes without volumes");
+  const uint32_t lane = threadIdx.x & 63u;
+  const float iw = 1.0f / (float)f.width, ih = 1.0f / (float)f.height;
+  const int spp = max(r.pixel_samples, 1);
+  const int aos = min(max(r.ambient_samples, 0), 256);
+  const int nl = KIND == VRX_RENDER_DIRECT ? (int)sc.num_lights : 0;
+  const int per = aos + nl; // secondary rays of a shading point
+  const bool cull = r.cull_backfaces != 0;
+  Pcg rs;
+  pcg_seed(rs, (uint64_t)px + (uint64_t)py * f.width, (uint64_t)f.frame_id);
+  float4 accum = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+  float dcur = FLT_MAX;
+  uint32_t pid = 0, oid = 0, iid = 0;
+  bool ids_changed = f.frame_id == 0;
+  if (inside && f.frame_id != 0) {
+    accum = ((const float4 *)f.d_accum)[idx];
+    if (f.d_depth)
+      dcur = f.d_depth[idx];
+  }
+  // samples whose secondary rays wait in the queue: each took `per` slots, its
+  // hit lanes are opaque at the first layer, the others missed
+  int pending = 0;
+  uint32_t hit_mask = 0;  // bit p: this lane hit in pending sample p
+  uint32_t valid = 0;     // bit slot: this lane queued a ray there
+  q.n = 0;
+
+  // results of the pending samples, oldest first
+  const auto resolve = [&](int count) {
+    for (int p = 0; p < count; p++) {
+      v3 outc = mk(0.0f, 0.0f, 0.0f);
+      float outo = 0.0f;
+      if ((hit_mask >> p) & 1u) {
+        const v3 scol = mk(gld(queue_sample(q, p, 0), lane), gld(queue_sample(q, p, 1), lane),
+            gld(queue_sample(q, p, 2), lane));
+        const float sop = gld(queue_sample(q, p, 3), lane);
+        SecondarySum s;
+        s.weights = s.hits = 0.0f;
+        s.contrib = mk(0.0f, 0.0f, 0.0f);
+        if (KIND == VRX_RENDER_DIRECT && r.ambient_radiance > 0.0f)
+          s.contrib = mulv(mulf(ld3(r.ambient_color), r.ambient_radiance), scol);
+        add_secondary<KIND>(sc, q, (uint32_t)(p * per), lane, 0, per, aos, valid, s);
+        shade_layer<KIND>(r, s, aos, scol, sop, outc, outo);
+      } else {
+        shade_miss(r, outc, outo);
+      }
+      if (inside)
+        add_sample(outc, outo, accum);
+    }
+  };
+
+  for (int sample = 0; sample < spp; sample++) {
+    v3 o = mk(0.0f, 0.0f, 0.0f), d = o;
+    if (inside) {
+      const float r0 = pcg_float(rs), r1 = pcg_float(rs);
+      (void)pcg_float(rs);
+      (void)pcg_float(rs);
+      cam_ray(cam, ((float)px + r0) * iw, ((float)py + r1) * ih, o, d);
+    }
+    float tlower = 0.0f, outo = 0.0f;
+    v3 outc = mk(0.0f, 0.0f, 0.0f);
+    bool alive = inside, deferred = false;
+    for (int layer = 0; layer < kMaxSurfaceLayers && __ballot(alive) != 0ull; layer++) {
+      // 1. the closest surface
+      bool hit = false;
+      v3 hp = mk(0.0f, 0.0f, 0.0f), ns = hp, scol = hp, ao_o = hp, sh_o = hp;
+      float sop = 0.0f;
+      if (alive) {
+        Hit h;
+        rays++;
+        hit = trace<PT, TWO, false, 2>(sc, o, d, tlower, FLT_MAX, cull, st, h);
+        float depth = 1e30f;
+        uint32_t prim = 0, obj = ~0u, inst = ~0u;
+        if (hit) {
+          SurfHit s;
+          populate(sc, h, o, d, s);
+          depth = s.t;
+          prim = s.prim_out;
+          obj = s.obj;
+          inst = s.inst;
+          hp = s.hp;
+          ns = s.ns;
+          scol = s.color;
+          sop = s.opacity;
+          ao_o = add(s.hp, fmul(s.eps, s.ng));
+          sh_o = add(s.hp, fmul(s.eps, s.ns));
+          tlower = s.t + s.eps;
+        }
+        if (layer == 0 && depth < dcur) {
+          dcur = depth;
+          pid = prim;
+          oid = obj;
+          iid = inst;
+          ids_changed = true;
+        }
+      }
+      // 2. its secondary rays, kQueueSlots at a time
+      const bool single = per <= kQueueSlots;
+      const bool wait =
+          layer == 0 && single && __ballot(hit && !(sop >= 0.99f && sop <= 1.0f)) == 0ull;
+      SecondarySum s;
+      s.weights = s.hits = 0.0f;
+      s.contrib = mk(0.0f, 0.0f, 0.0f);
+      if (KIND == VRX_RENDER_DIRECT && r.ambient_radiance > 0.0f)
+        s.contrib = mulv(mulf(ld3(r.ambient_color), r.ambient_radiance), scol);
+      if (!wait && pending > 0) {
+        queue_drain<PT, TWO>(sc, q, lane, st);
+        resolve(pending);
+        pending = 0;
+        hit_mask = valid = 0;
+      }
+      const v3 kd = mulf(scol, 0.318309886183790672f);
+      const uint32_t base = (uint32_t)(pending * per);
+      for (int k0 = 0; k0 < per; k0 += kQueueSlots) {
+        const int k1 = min(k0 + kQueueSlots, per);
+        for (int k = k0; k < k1; k++) {
+          const uint32_t slot = base + (uint32_t)(k - k0);
+          v3 dir = mk(0.0f, 0.0f, 1.0f), w = mk(0.0f, 0.0f, 0.0f);
+          float tmax = r.ao_distance;
+          bool queue = false;
+          if (k < aos) {
+            // computeAO, as in ao_factor()
+            if (hit) {
+              float q0 = pcg_float(rs), q1 = pcg_float(rs), q2 = pcg_float(rs);
+              (void)pcg_float(rs);
+              dir = normalize(mk(2.0f * q0 - 1.0f, 2.0f * q1 - 1.0f, 2.0f * q2 - 1.0f));
+              if (!(dot(dir, ns) > 0.0f))
+                dir = neg(dir);
+              w.x = fmaxf(0.0f, dot(dir, ns));
+              queue = w.x != 0.0f;
+            }
+          } else if (KIND == VRX_RENDER_DIRECT && hit) {
+            // as in shade_direct()
+            const LightSample ls = sample_light(sc.d_lights + (k - aos), hp);
+            const float ndl = fmaxf(0.0f, dot(ns, ls.dir));
+            w = mulv(mulf(kd, ndl), ls.radiance);
+            dir = ls.dir;
+            tmax = ls.dist;
+            queue = !(w.x != w.x || w.y != w.y || w.z != w.z)
+                && !(w.x == 0.0f && w.y == 0.0f && w.z == 0.0f);
+          }
+          if (queue) {
+            rays++;
+            valid |= 1u << slot;
+          }
+          queue_push(q, slot, lane, queue, k < aos ? ao_o : sh_o, dir, w, tmax);
+        }
+        if (!wait) {
+          queue_drain<PT, TWO>(sc, q, lane, st);
+          if (hit)
+            add_secondary<KIND>(sc, q, 0u, lane, k0, k1, aos, valid, s);
+          valid = 0;
+        }
+      }
+      // 3. the layer
+      if (wait) {
+        if (hit) {
+          gst(queue_sample(q, pending, 0), lane, scol.x);
+          gst(queue_sample(q, pending, 1), lane, scol.y);
+          gst(queue_sample(q, pending, 2), lane, scol.z);
+          gst(queue_sample(q, pending, 3), lane, sop);
+          hit_mask |= 1u << pending;
+        }
+        pending++;
+        deferred = true;
+        break;
+      }
+      if (alive) {
+        if (hit) {
+          shade_layer<KIND>(r, s, aos, scol, sop, outc, outo);
+          alive = outo < 0.99f;
+        } else {
+          shade_miss(r, outc, outo);
+          alive = false;
+        }
+      }
+    }
+    if (!deferred) {
+      if (inside)
+        add_sample(outc, outo, accum);
+    } else if ((pending + 1) * per > kQueueSlots || pending >= kQueueSlots || sample + 1 == spp) {
+      queue_drain<PT, TWO>(sc, q, lane, st);
+      resolve(pending);
+      pending = 0;
+      hit_mask = valid = 0;
+    }
+  }
+  if (inside)
+    write_pixel(f, idx, accum, spp, dcur, ids_changed, pid, oid, iid);
+}
+
+// --------------------------------------------------------------------------
 // the per-pixel program
 // --------------------------------------------------------------------------
 // One pixel of the raycast / AO / directLight program (Raycast_ptx.cu:60-179,

@@ -664,14 +664,16 @@ __device__ __forceinline__ bool visit4(const Node4 &nd, v3 o, v3 inv, float tmin
   return true;
 }
 
-// Reciprocal directions for the packed nodes' plane distances: a zero
-// direction component gives 2^100 instead of infinity, so that a plane
-// through the grid origin does not become 0 * infinity.
+// Reciprocal directions for the packed nodes' plane distances, by v_rcp_f32
+// (one ulp, within the slack below): a zero direction component gives 2^100
+// instead of infinity, so that a plane through the grid origin does not become
+// 0 * infinity.
 __device__ __forceinline__ v3 pack_inv(v3 d)
 {
   constexpr float big = 0x1p100f;
-  return mk(fminf(fmaxf(1.0f / d.x, -big), big), fminf(fmaxf(1.0f / d.y, -big), big),
-      fminf(fmaxf(1.0f / d.z, -big), big));
+  return mk(__builtin_amdgcn_fmed3f(__builtin_amdgcn_rcpf(d.x), -big, big),
+      __builtin_amdgcn_fmed3f(__builtin_amdgcn_rcpf(d.y), -big, big),
+      __builtin_amdgcn_fmed3f(__builtin_amdgcn_rcpf(d.z), -big, big));
 }
 
 // slack of the packed slab test, on the far side alone: the 2^-18 of slab()
@@ -711,13 +713,30 @@ __device__ __forceinline__ void slab4p(const Node4p &nd, v3 o, v3 inv, float tmi
   }
 }
 
-// visit4() on a packed node
+// visit4() on a packed node.  Any-hit walks take the children as they come:
+// sorting them costs more than the order saves (1M lit spheres 3.82 -> 3.70 ms,
+// AO on 10M spheres unchanged).
+template <bool ANY>
 __device__ __forceinline__ bool visit4p(const Node4p &nd, v3 o, v3 inv, float tmin, float tmax,
     Stack &st, uint32_t &node)
 {
   uint32_t l[4] = {nd.link.x, nd.link.y, nd.link.z, nd.link.w};
   float t[4];
   slab4p(nd, o, inv, tmin, tmax, t);
+  if (ANY) {
+    bool have = false;
+#pragma unroll
+    for (int c = 0; c < 4; c++) {
+      if (t[c] < INFINITY) {
+        if (have)
+          st.push(l[c]);
+        else
+          node = l[c];
+        have = true;
+      }
+    }
+    return have;
+  }
   cswap(t[0], l[0], t[1], l[1]);
   cswap(t[2], l[2], t[3], l[3]);
   cswap(t[0], l[0], t[2], l[2]);
@@ -808,7 +827,7 @@ __device__ bool trace(const vrx_scene &sc, v3 wo, v3 wd, float tmin, float tmax,
     bool do_pop = true;
     if (WIDE == 2 && !(node & kLeafBit)) {
       const Node4p nd = gld_node4p((const Node4p *)wnodes, node);
-      do_pop = !visit4p(nd, o, inv, tmin, h.t, st, node);
+      do_pop = !visit4p<ANY>(nd, o, inv, tmin, h.t, st, node);
     } else if (WIDE == 2 && node == kPackEmpty) {
       // an unused slot, "hit" where rounding swallows the whole grid
     } else if (WIDE == 1 && !(node & kLeafBit)) {
@@ -878,6 +897,131 @@ __device__ bool trace(const vrx_scene &sc, v3 wo, v3 wd, float tmin, float tmax,
     }
   }
 }
+
+// A walk advanced a step at a time (packed nodes), for waves whose lanes take
+// their next ray when one ends.  attach() loads what all rays share; begin()
+// starts a ray; step() returns true at the ray's end, with the closest hit in
+// h or, ANY, the opacity met in h.a0.
+template <int PT, bool TWO, bool ANY>
+struct Walk {
+  v3 o, d, inv;       // the ray in the space of the current nodes
+  v3 wo, wd, winv;    // the ray in world space (TWO)
+  float tmin;
+  uint32_t node;
+  const void *nodes;
+  BlasCtx b;
+  WT wt;
+  bool in_blas;
+  Hit h;
+
+  __device__ __forceinline__ bool attach(const vrx_scene &sc, bool cull_all)
+  {
+    if (sc.num_entries == 0)
+      return false;
+    if constexpr (!TWO) {
+      uint32_t n;
+      v3 uo, ud;
+      load_blas(sc, 0u, mk(0.0f, 0.0f, 0.0f), mk(0.0f, 0.0f, 0.0f), cull_all, ANY, b, uo, ud,
+          node, n);
+      return n != 0;
+    }
+    return true;
+  }
+
+  __device__ __forceinline__ void leave(const vrx_scene &sc)
+  {
+    in_blas = false;
+    nodes = sc.tlas.d_wide;
+    o = wo;
+    d = wd;
+    inv = winv;
+  }
+
+  __device__ __forceinline__ void begin(const vrx_scene &sc, v3 ro, v3 rd, float t0, float t1,
+      Stack &st)
+  {
+    h.found = false;
+    h.entry = h.prim = 0;
+    h.a0 = h.a1 = h.a2 = 0.0f;
+    h.t = t1;
+    tmin = t0;
+    st.cnt = 0;
+    if constexpr (TWO) {
+      wo = ro;
+      wd = rd;
+      winv = pack_inv(rd);
+      leave(sc);
+      node = sc.num_entries == 1 ? kLeafBit : 0u;
+    } else {
+      const vrx_entry *E = sc.d_entries;
+      o = ro;
+      d = rd;
+      if (!gld(&E->identity)) {
+        float m[12];
+#pragma unroll
+        for (int q = 0; q < 12; q++)
+          m[q] = gld(&E->inv[q]);
+        o = xfm_point(m, ro);
+        d = xfm_vector(m, rd);
+      }
+      inv = pack_inv(d);
+      if (blas_type<PT>(b) == VRX_TRIANGLE)
+        wt = wt_setup(d);
+      nodes = b.wnodes;
+      node = b.boxed ? 0u : kLeafBit;
+    }
+  }
+
+  __device__ __forceinline__ bool step(const vrx_scene &sc, bool cull_all, Stack &st)
+  {
+    bool do_pop = true;
+    if (!(node & kLeafBit)) {
+      const Node4p nd = gld_node4p((const Node4p *)nodes, node);
+      do_pop = !visit4p<ANY>(nd, o, inv, tmin, h.t, st, node);
+    } else if (node == kPackEmpty) {
+      // an unused slot, "hit" where rounding swallows the whole grid
+    } else if (!TWO || in_blas) {
+      BoxGuard<TWO> guard;
+      if constexpr (TWO) {
+        guard.entry_box = (const float *)((const Node4p *)sc.tlas.d_wide + (sc.num_entries - 1));
+        guard.wo = wo;
+        guard.wd = wd;
+      }
+      float tcur = h.t;
+      if (test_leaf<PT, ANY>(b, node & ~kLeafBit, o, d, wt, tmin, tcur, h, guard))
+        return true;
+    } else {
+      uint32_t n, root;
+      load_blas(sc, gld(sc.tlas.d_leaf_ids, node & ~kLeafBit), wo, wd, cull_all, ANY, b, o, d, root, n);
+      if (n != 0) {
+        inv = pack_inv(d);
+        if (blas_type<PT>(b) == VRX_TRIANGLE)
+          wt = wt_setup(d);
+        st.push(kMarker);
+        in_blas = true;
+        nodes = b.wnodes;
+        node = root;
+        do_pop = false;
+      } else {
+        o = wo;
+        d = wd;
+      }
+    }
+    if (do_pop) {
+      for (;;) {
+        if (st.cnt == 0)
+          return true;
+        node = st.pop();
+        if (TWO && node == kMarker) {
+          leave(sc);
+          continue;
+        }
+        break;
+      }
+    }
+    return false;
+  }
+};
 
 // Surface hit in world space (populateHit.h:150-368).
 struct SurfHit {
