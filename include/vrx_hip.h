@@ -133,8 +133,8 @@ int vrx_bvh_widen(const vrx_bvh *bvh, uint32_t n, vrx_stream s);
  * grid over the record's box, rounded outwards; the traversal checks a hit
  * against its exact leaf box, so frames do not depend on the node format.
  * Writes bvh->d_wide, which must hold vrx_bvh_packed_bytes(type, n); type is
- * the primitive type of the build (VRX_BOX: the instance level, which also
- * stores its n entry boxes). */
+ * the primitive type of the build.  The instance level (VRX_BOX) is packed by
+ * vrx_tlas_pack, which also writes a 128-byte record per instance. */
 size_t vrx_bvh_packed_bytes(int32_t type, uint32_t n);
 int vrx_bvh_pack(const vrx_bvh *bvh, int32_t type, uint32_t n, vrx_stream s);
 /* Debug/parity hooks: read back the sorted Morton codes (n) and the order. */
@@ -245,6 +245,10 @@ typedef struct vrx_scene {
                                    vrx_bvh_pack; any other value = by vrx_bvh_widen */
 } vrx_scene;
 #define VRX_WIDE_PACKED 0x34503634u
+/* Packed nodes and instance records of scene->tlas (num_entries > 1), into
+ * tlas.d_wide, which must hold vrx_bvh_packed_bytes(VRX_BOX, num_entries).
+ * Reads the entries and geometries, whose d_wide must already be packed. */
+int vrx_tlas_pack(const vrx_scene *scene, vrx_stream s);
 
 typedef struct vrx_camera {
   float pos[3];

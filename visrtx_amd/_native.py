@@ -176,6 +176,7 @@ def hip() -> C.CDLL:
             "vrx_bvh_widen": (i32, [vp, u32, vp]),
             "vrx_bvh_packed_bytes": (sz, [i32, u32]),
             "vrx_bvh_pack": (i32, [vp, i32, u32, vp]),
+            "vrx_tlas_pack": (i32, [vp, vp]),
             "vrx_render_scratch_bytes": (sz, [vp, vp, u32, u32]),
             "vrx_frame_clear": (i32, [vp, vp]),
             "vrx_render": (i32, [vp, vp, vp, vp, vp]),

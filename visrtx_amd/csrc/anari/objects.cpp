@@ -1611,17 +1611,17 @@ int World::ensureWide()
       return -1;
     hostGeoms[i].bvh.d_wide = g->dWide;
   }
-  if (scene.num_entries > 1) {
-    scene.tlas.d_wide = dTlasWide;
-    if (!dev->check(vrx_bvh_pack(&scene.tlas, VRX_BOX, scene.num_entries, s), this, "4-wide instance nodes"))
-      return -1;
-  }
-  vrx_event_record(e1, s);
   if (!hostGeoms.empty()
       && !dev->check(vrx_memcpy(dGeoms, hostGeoms.data(), hostGeoms.size() * sizeof(vrx_geom),
                          VRX_H2D, s),
           this, "scene upload"))
     return -1;
+  if (scene.num_entries > 1) {
+    scene.tlas.d_wide = dTlasWide;
+    if (!dev->check(vrx_tlas_pack(&scene, s), this, "4-wide instance nodes"))
+      return -1;
+  }
+  vrx_event_record(e1, s);
   dev->check(vrx_stream_sync(s), this, "stream sync");
   float ms = 0.0f;
   vrx_event_elapsed_ms(e0, e1, &ms);

@@ -1277,11 +1277,7 @@ __device__ __forceinline__ bool pack_axis(const PackSlot s[4], uint32_t cnt, int
   return fin;
 }
 
-// LEAF_BOX: also store the exact box of every leaf by its primitive (the
-// instance level: entry boxes, which have no leaf record to derive them from)
-template <bool LEAF_BOX>
-__global__ __launch_bounds__(256) void k_pack(const Node *nodes, uint32_t ninner, Node4p *out,
-    const uint32_t *leaf_ids, float *leaf_box)
+__global__ __launch_bounds__(256) void k_pack(const Node *nodes, uint32_t ninner, Node4p *out)
 {
   const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= ninner)
@@ -1290,16 +1286,6 @@ __global__ __launch_bounds__(256) void k_pack(const Node *nodes, uint32_t ninner
   const Node nd = gld_node(nodes, i);
   node_child(nd, 0, s[0].b, s[0].link);
   node_child(nd, 1, s[1].b, s[1].link);
-  if constexpr (LEAF_BOX) {
-#pragma unroll
-    for (int j = 0; j < 2; j++)
-      if (s[j].link & kLeafBit) {
-        float *b = leaf_box + 6 * (size_t)gld(leaf_ids, s[j].link & ~kLeafBit);
-#pragma unroll
-        for (int q = 0; q < 6; q++)
-          gst(b, q, s[j].b[q]);
-      }
-  }
   const bool in0 = !(s[0].link & kLeafBit), in1 = !(s[1].link & kLeafBit);
   uint32_t cnt = 2;
   s[2] = s[3] = s[1];
@@ -1472,6 +1458,18 @@ int bvh_build_impl(const vrx_prims *p, const vrx_bvh *out, void *d_ws, size_t ws
   }
 }
 
+int bvh_pack_impl(const vrx_bvh *bvh, uint32_t n, hipStream_t s)
+{
+  if (n < 2)
+    return VRX_OK; // a single leaf (or nothing): no inner nodes
+  VRX_ARG(bvh->d_nodes && bvh->d_wide, "bvh nodes / packed buffer");
+  const uint32_t ninner = n - 1;
+  hipLaunchKernelGGL(k_pack, dim3((ninner + 255) / 256), dim3(256), 0, s,
+      (const Node *)bvh->d_nodes, ninner, (Node4p *)bvh->d_wide);
+  VRX_LAUNCH_CHECK();
+  return VRX_OK;
+}
+
 void bvh_sizes(int32_t type, uint32_t n, vrx_bvh_sizes *o)
 {
   o->nodes = (size_t)(n > 1 ? n - 1 : 1) * sizeof(Node);
@@ -1512,28 +1510,15 @@ size_t vrx_bvh_packed_bytes(int32_t type, uint32_t n)
 {
   if (n < 2)
     return 0;
-  return (size_t)(n - 1) * sizeof(Node4p) + (type == VRX_BOX ? (size_t)n * 24 : 0);
+  return type == VRX_BOX ? inst_rec_offset(n) + (size_t)n * sizeof(InstRec)
+                         : (size_t)(n - 1) * sizeof(Node4p);
 }
 
 int vrx_bvh_pack(const vrx_bvh *bvh, int32_t type, uint32_t n, vrx_stream s)
 {
   VRX_ARG(bvh, "bvh");
-  VRX_ARG(type >= 0 && type <= VRX_CURVE, "type");
-  if (n < 2)
-    return VRX_OK; // a single leaf (or nothing): no inner nodes
-  VRX_ARG(bvh->d_nodes && bvh->d_wide, "bvh nodes / packed buffer");
-  VRX_ARG(type != VRX_BOX || bvh->d_leaf_ids, "leaf ids");
-  const uint32_t ninner = n - 1;
-  const dim3 grid((ninner + 255) / 256);
-  Node4p *out = (Node4p *)bvh->d_wide;
-  if (type == VRX_BOX)
-    hipLaunchKernelGGL(k_pack<true>, grid, dim3(256), 0, (hipStream_t)s,
-        (const Node *)bvh->d_nodes, ninner, out, bvh->d_leaf_ids, (float *)(out + ninner));
-  else
-    hipLaunchKernelGGL(k_pack<false>, grid, dim3(256), 0, (hipStream_t)s,
-        (const Node *)bvh->d_nodes, ninner, out, (const uint32_t *)nullptr, (float *)nullptr);
-  VRX_LAUNCH_CHECK();
-  return VRX_OK;
+  VRX_ARG(type >= 0 && type <= VRX_CURVE && type != VRX_BOX, "type (instances: vrx_tlas_pack)");
+  return bvh_pack_impl(bvh, n, (hipStream_t)s);
 }
 
 size_t vrx_bvh_wide_bytes(uint32_t n)

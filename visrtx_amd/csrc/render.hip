@@ -629,16 +629,15 @@ __global__ __launch_bounds__(256) void k_sample_distance(vrx_volume v, uint32_t 
   out_albedo[3 * (size_t)i + 2] = alb.z;
 }
 
-__global__ void k_entry_boxes(vrx_scene sc, float *boxes)
+// world box of entry e
+__device__ __forceinline__ void entry_box(const vrx_scene &sc, uint32_t e, v3 &wlo, v3 &whi)
 {
-  uint32_t e = blockIdx.x * blockDim.x + threadIdx.x;
-  if (e >= sc.num_entries)
-    return;
   const vrx_entry &E = sc.d_entries[e];
   const vrx_geom &G = sc.d_geoms[E.geom];
   const vrx_bvh_header *H = (const vrx_bvh_header *)G.bvh.d_header;
   v3 lo = mk(H->lo[0], H->lo[1], H->lo[2]), hi = mk(H->hi[0], H->hi[1], H->hi[2]);
-  v3 wlo = lo, whi = hi;
+  wlo = lo;
+  whi = hi;
   if (!E.identity && G.n > 0) {
     wlo = mk(INFINITY, INFINITY, INFINITY);
     whi = mk(-INFINITY, -INFINITY, -INFINITY);
@@ -650,9 +649,49 @@ __global__ void k_entry_boxes(vrx_scene sc, float *boxes)
       whi = vmax(whi, q);
     }
   }
+}
+
+__global__ void k_entry_boxes(vrx_scene sc, float *boxes)
+{
+  uint32_t e = blockIdx.x * blockDim.x + threadIdx.x;
+  if (e >= sc.num_entries)
+    return;
+  v3 wlo, whi;
+  entry_box(sc, e, wlo, whi);
   float *b = boxes + 6 * (size_t)e;
   b[0] = wlo.x; b[1] = wlo.y; b[2] = wlo.z;
   b[3] = whi.x; b[4] = whi.y; b[5] = whi.z;
+}
+
+// the record of the instance at sorted leaf k of the instance level
+__global__ __launch_bounds__(256) void k_inst_records(vrx_scene sc, InstRec *out)
+{
+  const uint32_t k = blockIdx.x * blockDim.x + threadIdx.x;
+  if (k >= sc.num_entries)
+    return;
+  const uint32_t e = sc.tlas.d_leaf_ids[k];
+  const vrx_entry &E = sc.d_entries[e];
+  const vrx_geom &G = sc.d_geoms[E.geom];
+  InstRec r;
+#pragma unroll
+  for (int q = 0; q < 12; q++)
+    r.inv[q] = E.inv[q];
+  r.nodes = G.bvh.d_wide;
+  r.leaves = G.bvh.d_leaves;
+  r.ids = G.bvh.d_leaf_ids;
+  r.entry = e;
+  r.flags = (E.identity ? kInstIdentity : 0u) | (G.n > 1 ? kInstBoxed : 0u)
+      | (G.cull_backfaces ? kInstCull : 0u) | (G.caps ? kInstCaps : 0u) | (G.n == 0 ? kInstEmpty : 0u)
+      | ((uint32_t)G.type << 8);
+  v3 lo, hi;
+  entry_box(sc, e, lo, hi);
+  r.box[0] = lo.x; r.box[1] = lo.y; r.box[2] = lo.z;
+  r.box[3] = hi.x; r.box[4] = hi.y; r.box[5] = hi.z;
+  r.opacity = G.opacity;
+#pragma unroll
+  for (int q = 0; q < 5; q++)
+    r.pad[q] = 0u;
+  out[k] = r;
 }
 
 // --------------------------------------------------------------------------
@@ -1067,6 +1106,20 @@ int vrx_tlas_query_sizes(uint32_t num_entries, vrx_bvh_sizes *out)
   VRX_ARG(out, "out");
   bvh_sizes(VRX_BOX, num_entries, out);
   out->workspace += ((size_t)num_entries * 24 + 255) & ~size_t(255);
+  return VRX_OK;
+}
+
+int vrx_tlas_pack(const vrx_scene *scene, vrx_stream s)
+{
+  VRX_ARG(scene && scene->d_entries && scene->d_geoms, "scene arrays");
+  VRX_ARG(scene->num_entries < 2 || scene->tlas.d_leaf_ids, "instance BVH not built");
+  const int st = bvh_pack_impl(&scene->tlas, scene->num_entries, (hipStream_t)s);
+  if (st || scene->num_entries < 2)
+    return st;
+  InstRec *rec = (InstRec *)((char *)scene->tlas.d_wide + inst_rec_offset(scene->num_entries));
+  hipLaunchKernelGGL(k_inst_records, dim3((scene->num_entries + 255) / 256), dim3(256), 0,
+      (hipStream_t)s, *scene, rec);
+  VRX_LAUNCH_CHECK();
   return VRX_OK;
 }
 

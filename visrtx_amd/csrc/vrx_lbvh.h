@@ -105,6 +105,30 @@ __device__ __forceinline__ Node4p gld_node4p(const Node4p *nodes, size_t i)
   return n;
 }
 
+// What a walk needs of an instance, one 128-byte line, in the order of the
+// instance level's sorted leaves (after its packed nodes): entering an
+// instance is one fetch instead of a chain of three (leaf id, entry,
+// geometry), and hits read the rest.
+struct alignas(128) InstRec {
+  float inv[12];          // world -> object
+  const void *nodes;      // packed nodes of the geometry
+  const void *leaves;
+  const uint32_t *ids;
+  uint32_t entry, flags;  // kInst* | type << 8
+  float box[6];           // the entry's exact box
+  float opacity;
+  uint32_t pad[5];
+};
+static_assert(sizeof(InstRec) == 128, "InstRec must be 128 bytes");
+constexpr uint32_t kInstIdentity = 1, kInstBoxed = 2, kInstCull = 4, kInstCaps = 8, kInstEmpty = 16;
+
+__host__ __device__ __forceinline__ size_t inst_rec_offset(uint32_t n)
+{
+  return ((size_t)(n - 1) * sizeof(Node4p) + 127) & ~size_t(127);
+}
+
+int bvh_pack_impl(const vrx_bvh *bvh, uint32_t n, hipStream_t s);
+
 // float4s per leaf record
 template <int T>
 constexpr int record_quads()
