@@ -1,0 +1,56 @@
+"""The forward's layouts: tiles of whole images, rays in no order, and the
+y-pair gathers that 65,536 rays and more take.  All sample the same positions
+in the same order, so a ray's colour and opacity are bit-identical; the
+gradients of a loss over all rays differ by the order of their 32-bit sums."""
+import numpy as np
+import pytest
+import torch
+
+from visrtx_amd import diffvol as D
+from visrtx_amd import scenes as S
+
+pytestmark = pytest.mark.gpu
+
+
+def _setup(dims, image):
+    nx, ny, nz = dims
+    sp = tuple(1.0 / (m - 1) for m in dims)
+    m = min(sp)
+    dens = torch.from_numpy(S.gen_noise_volume(nx, ny, nz, seed=4)).cuda()
+    lut = torch.from_numpy(D.colormap_lut(S.COLORMAP5, np.array([0.0, 0.4]))).cuda()
+    views = -(-66_000 // (image[0] * image[1]))
+    org, dirs = D.make_rays(D.orbit_cameras(views, seed=3, fovy=45.0), *image)
+    spec = dict(dims=dims, spacing=sp, unit_distance=m, step=0.5 * m)
+    return dens, lut, org, dirs, spec
+
+
+@pytest.mark.parametrize("dims", [(2, 2, 2), (17, 9, 33), (64, 64, 64), (65, 2, 31)])
+@pytest.mark.parametrize("image", [(255, 263), (23, 17), (64, 64)])
+def test_layouts_give_the_same_rays(require_gpu, dims, image):
+    dens, lut, org, dirs, spec = _setup(dims, image)
+    print(f"[forward] {dims} {image} {len(org)} rays", flush=True)
+    with torch.no_grad():
+        whole = D.render(dens, lut, org, dirs, D.GridSpec(**spec, image=image))
+        loose = D.render(dens, lut, org, dirs, D.GridSpec(**spec))
+        parts = torch.cat([D.render(dens, lut, o.contiguous(), d.contiguous(), D.GridSpec(**spec))
+                           for o, d in zip(org.split(30_011), dirs.split(30_011))])
+        # an image size that does not divide the rays is a hint that does not apply
+        odd = D.render(dens, lut, org, dirs, D.GridSpec(**spec, image=(image[0] + 1, image[1] + 2)))
+    torch.cuda.synchronize()
+    for other in (loose, parts, odd):
+        assert torch.equal(whole, other)
+    assert (whole[:, 3] > 0).any()
+
+
+def test_gradients_of_many_rays(require_gpu):
+    dens, lut, org, dirs, spec = _setup((33, 20, 27), (64, 64))
+    up = torch.randn((len(org), 4), device="cuda", generator=torch.Generator("cuda").manual_seed(1))
+    got = []
+    for n in (len(org), 20_480):
+        d, l = dens.clone().requires_grad_(True), lut.clone().requires_grad_(True)
+        for o, v, g in zip(org.split(n), dirs.split(n), up.split(n)):
+            D.render(d, l, o.contiguous(), v.contiguous(),
+                     D.GridSpec(**spec, image=(64, 64))).backward(g.contiguous())
+        got.append((d.grad, l.grad))
+    for a, b in zip(*got):
+        assert float((a - b).norm() / b.norm()) < 2e-5
