@@ -191,7 +191,8 @@ typedef struct vrx_volume {
   float unit_distance;
   uint32_t id;
   uint32_t inst_id;
-  uint32_t pad;
+  uint32_t grid_format;   /* VRX_GRID_DISTANCES: d_majorant is followed by the cells'
+                             distances (vrx_volume_grid_distances); else it is not */
   /* NULL, or the macro-cell majorant grid from vrx_volume_majorant_grid: the
    * march skips the samples inside cells whose majorant is 0 (they add
    * nothing), when the renderer's skip_empty is set */
@@ -203,6 +204,7 @@ typedef struct vrx_volume {
    * under 2^29 voxels and under 2^24 rows); same values, same frame */
   const float *d_ypairs;
 } vrx_volume;
+#define VRX_GRID_DISTANCES 0x64737431u
 
 /* One light in world space, as the directLight renderer samples it
  * (gpu/sampleLight.h:58-100; scene/light/{Directional,Point,Spot}.cpp).
@@ -343,6 +345,14 @@ int vrx_render(const vrx_scene *scene, const vrx_camera *cam, const vrx_renderer
  * vrx_volume_grid_cells(v) floats, x fastest; v->d_data and v->d_lut are read. */
 size_t vrx_volume_grid_cells(const vrx_volume *v);
 int vrx_volume_majorant_grid(const vrx_volume *v, float *d_majorant, vrx_stream s);
+/* Appends to a majorant grid the distance of every cell to the nearest cell
+ * with a majorant above 0, in cells of the larger axis offset (0 there, at
+ * most 255; the grid's surroundings count as empty): one byte per cell right
+ * after the vrx_volume_grid_cells(v) majorants.  The march then leaves an
+ * empty cell together with all cells nearer than that in one step.  d_grid
+ * must hold vrx_volume_grid_bytes(v) (it is also used as work space). */
+size_t vrx_volume_grid_bytes(const vrx_volume *v);
+int vrx_volume_grid_distances(const vrx_volume *v, float *d_grid, vrx_stream s);
 /* Writes v's field as y-pairs (see vrx_volume.d_ypairs) to d_ypairs, which
  * holds dims[0]*dims[1]*dims[2] float2.  No reference counterpart (the
  * reference samples a CUDA 3D texture, whose layout the driver chooses); the

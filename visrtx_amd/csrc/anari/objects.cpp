@@ -1469,7 +1469,7 @@ int World::rebuild()
         vrx_free(v->dGrid);
         v->dGrid = nullptr;
         v->gridCells = 0;
-        if (dev->check(vrx_malloc(&v->dGrid, cells * sizeof(float)), this, "majorant grid"))
+        if (dev->check(vrx_malloc(&v->dGrid, vrx_volume_grid_bytes(&vv)), this, "majorant grid"))
           v->gridCells = cells;
       }
       std::vector<float> mg(cells);
@@ -1480,8 +1480,12 @@ int World::rebuild()
           && dev->check(vrx_stream_sync(s), this, "stream sync")) {
         const size_t empty = (size_t)std::count(mg.begin(), mg.end(), 0.0f);
         v->emptyCellFraction = cells ? (float)empty / (float)cells : 0.0f;
-        if (8 * empty >= cells && empty > 0)
+        if (8 * empty >= cells && empty > 0) {
           vv.d_majorant = (const float *)v->dGrid;
+          if (dev->check(vrx_volume_grid_distances(&vv, (float *)v->dGrid, s), this,
+                  "majorant grid"))
+            vv.grid_format = VRX_GRID_DISTANCES;
+        }
       }
     }
     // a dense field alone in its world is marched by the four-lane kernel,

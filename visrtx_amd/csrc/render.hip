@@ -546,6 +546,34 @@ __global__ __launch_bounds__(256) void k_majorants(vrx_volume v, float *out)
   out[cell] = m;
 }
 
+// One axis of the cells' Chebyshev distance to the nearest cell that is not
+// empty, min over the row of max(offset, the distance over the axes before);
+// AXIS 0 reads the majorants.  A few cells' loads per cell, once per world
+// build.
+template <int AXIS>
+__global__ __launch_bounds__(256) void k_grid_distance(const float *majorant, const uint8_t *in,
+    uint8_t *out, int mx, int my, int mz)
+{
+  const int i = (int)(blockIdx.x * blockDim.x + threadIdx.x);
+  if (i >= mx * my * mz)
+    return;
+  const int c[3] = {i % mx, (i / mx) % my, i / (mx * my)};
+  const int len = AXIS == 0 ? mx : AXIS == 1 ? my : mz;
+  const int stride = AXIS == 0 ? 1 : AXIS == 1 ? mx : mx * my;
+  const int at = c[AXIS];
+  const auto dist = [&](int j) {
+    return AXIS == 0 ? (gld(majorant + j) == 0.0f ? 255 : 0) : (int)gld(in + j);
+  };
+  int best = dist(i);
+  for (int k = 1; k < best && (at - k >= 0 || at + k < len); k++) {
+    if (at - k >= 0)
+      best = min(best, max(k, dist(i - k * stride)));
+    if (at + k < len)
+      best = min(best, max(k, dist(i + k * stride)));
+  }
+  out[i] = (uint8_t)best;
+}
+
 // Woodcock (delta) tracking of one ray per lane through a volume with a
 // majorant grid (volumeIntegration.h:167-228 with dda.h:43-122): the ray
 // walks the 16^3-voxel macro cells it crosses; in a cell of majorant m it
@@ -950,7 +978,7 @@ int vrx_render(const vrx_scene *scene, const vrx_camera *cam, const vrx_renderer
       // dense field: four lanes per ray, volumeUnroll blocks of four samples
       // per iteration (default 2)
       dim3 grid((f->width + kVolTile - 1) / kVolTile, (f->height + kVolTile - 1) / kVolTile);
-      const int u = r->vol_unroll > 0 ? r->vol_unroll : 2;
+      const int u = r->vol_unroll > 0 ? r->vol_unroll : 4;
 #define VRX_VOL_LAUNCH(B, U)                                                                    \
   hipLaunchKernelGGL((k_render_volume_quad<B, U>), grid, dim3(kBlock), 0, st, *scene, *cam, *r, \
       *f)
@@ -1058,6 +1086,31 @@ int vrx_volume_majorant_grid(const vrx_volume *v, float *d_majorant, vrx_stream 
   VRX_ARG(cells < (1u << 31), "too many macro cells");
   hipLaunchKernelGGL(k_majorants, dim3((unsigned)cells), dim3(256), 0, (hipStream_t)s, *v,
       d_majorant);
+  VRX_LAUNCH_CHECK();
+  return VRX_OK;
+}
+
+size_t vrx_volume_grid_bytes(const vrx_volume *v)
+{
+  // majorants, distances, and the distances over fewer axes
+  return vrx_volume_grid_cells(v) * (sizeof(float) + 2);
+}
+
+int vrx_volume_grid_distances(const vrx_volume *v, float *d_grid, vrx_stream s)
+{
+  VRX_ARG(v && d_grid, "null argument");
+  const size_t cells = vrx_volume_grid_cells(v);
+  VRX_ARG(cells > 0 && cells < (1u << 31), "volume dims");
+  const int mx = ((int)v->dims[0] + 15) >> 4, my = ((int)v->dims[1] + 15) >> 4,
+            mz = ((int)v->dims[2] + 15) >> 4;
+  uint8_t *a = (uint8_t *)(d_grid + cells), *b = a + cells;
+  const dim3 grid((unsigned)((cells + 255) / 256));
+  hipLaunchKernelGGL(k_grid_distance<0>, grid, dim3(256), 0, (hipStream_t)s, d_grid,
+      (const uint8_t *)nullptr, a, mx, my, mz);
+  hipLaunchKernelGGL(k_grid_distance<1>, grid, dim3(256), 0, (hipStream_t)s, d_grid,
+      (const uint8_t *)a, b, mx, my, mz);
+  hipLaunchKernelGGL(k_grid_distance<2>, grid, dim3(256), 0, (hipStream_t)s, d_grid,
+      (const uint8_t *)b, a, mx, my, mz);
   VRX_LAUNCH_CHECK();
   return VRX_OK;
 }

@@ -69,6 +69,7 @@ struct VolCtx {
   uint32_t sy, sz;
   float step, expo, lo, hi, inv_range;
   const float *mc; // macro-cell majorants (16^3 voxels per cell) or null
+  const uint8_t *md; // the cells' distances to the nearest cell that is not empty, or null
   int mcd[3];
   // the 32-bit gather form (b32): the field has 2 to 2^24 - 1 voxels along x,
   // under 2^30 voxels and under 2^24 x-rows, so a voxel's byte offset fits
@@ -96,6 +97,8 @@ __device__ __forceinline__ VolCtx vol_ctx(const vrx_volume &v, float inv_rate, b
 #pragma unroll
   for (int k = 0; k < 3; k++)
     c.mcd[k] = ((int)v.dims[k] + 15) >> 4;
+  c.md = c.mc && v.grid_format == VRX_GRID_DISTANCES
+      ? (const uint8_t *)(c.mc + (size_t)c.mcd[0] * c.mcd[1] * c.mcd[2]) : nullptr;
 #pragma unroll
   for (int k = 0; k < 3; k++) {
     c.dims[k] = (int)v.dims[k];
@@ -333,7 +336,8 @@ __device__ __forceinline__ float4 classify_delta(const float4 *lut2, const VolCt
 // positions do not depend on the accumulation), which keeps 8*U loads in
 // flight per lane; samples past the exit or the 0.99 cut-off are discarded,
 // their clamped gathers always stay inside the field.
-template <bool I64, int U, bool LUT_GLOBAL, bool SKIP, int XP>
+// SKIP: 0 every sample, 1 over a grid of majorants, 2 over one with distances.
+template <bool I64, int U, bool LUT_GLOBAL, int SKIP, int XP>
 __device__ __forceinline__ void march_xp(const VolCtx &c, const float4 *lut, v3 o, v3 d, float t0,
     float t1, v3 &color, float &opacity, uint32_t &ns)
 {
@@ -344,13 +348,40 @@ __device__ __forceinline__ void march_xp(const VolCtx &c, const float4 *lut, v3 
   float T = 1.0f;
   // macro-cell walk: per axis the reciprocal direction in voxel units
   [[maybe_unused]] float ig[3] = {0.0f, 0.0f, 0.0f};
-  if constexpr (SKIP) {
+  if constexpr (SKIP != 0) {
     ig[0] = gdx != 0.0f ? 1.0f / gdx : 0.0f;
     ig[1] = gdy != 0.0f ? 1.0f / gdy : 0.0f;
     ig[2] = gdz != 0.0f ? 1.0f / gdz : 0.0f;
   }
   for (uint32_t k = 0; k < kMaxSamplesPerSegment; k += U) {
-    if (SKIP && c.mc) {
+    if constexpr (SKIP == 2) {
+      // an empty cell at distance D of the nearest other: the cube of cells
+      // nearer than D is empty, and the march goes on at the first sample
+      // past its exit.  One lookup a cube instead of one for two cells (see
+      // SKIP 1), each a dependent load: sparse 512^3 frame 355 -> 289 us.
+      const float t = t0 + (float)k * c.step;
+      if (!(t <= t1))
+        break;
+      const float gd[3] = {gdx, gdy, gdz}, go[3] = {gox, goy, goz};
+      int cc[3];
+#pragma unroll
+      for (int a = 0; a < 3; a++)
+        cc[a] = min(max((int)floorf((go[a] + gd[a] * t) * 0.0625f), 0), c.mcd[a] - 1);
+      const int dist = (int)gld(c.md + ((size_t)cc[2] * c.mcd[1] + cc[1]) * c.mcd[0] + cc[0]);
+      if (dist > 0) {
+        float te = INFINITY;
+#pragma unroll
+        for (int a = 0; a < 3; a++)
+          if (gd[a] != 0.0f)
+            te = fminf(te, (16.0f * (float)(cc[a] + (gd[a] > 0.0f ? dist : 1 - dist)) - go[a]) * ig[a]);
+        const float kn = ceilf((te - t0) / c.step);
+        if (!(kn < (float)kMaxSamplesPerSegment))
+          break;
+        k = max((uint32_t)fmaxf(kn, 0.0f), k + 1) - U;
+        continue;
+      }
+    }
+    if (SKIP == 1 && c.mc) {
       // empty-space skipping: a macro cell with a 0 majorant adds nothing
       // between the ray's entry and exit (alpha 0 gives a step transmittance
       // of exactly 1), so the march jumps to the first sample past the exit.
@@ -448,13 +479,18 @@ __device__ __forceinline__ void march_xp(const VolCtx &c, const float4 *lut, v3 
   }
 }
 
-template <bool I64, int U, bool LUT_GLOBAL, bool SKIP = true>
+template <bool I64, int U, bool LUT_GLOBAL, int SKIP = 1>
 __device__ __forceinline__ void march(const VolCtx &c, const float4 *lut, v3 o, v3 d, float t0,
     float t1, v3 &color, float &opacity, uint32_t &ns)
 {
   if (!(c.step > 0.0f))
     return;
-  if (c.dims[0] >= 2)
+  if (SKIP == 1 && c.md) {
+    if (c.dims[0] >= 2)
+      march_xp<I64, U, LUT_GLOBAL, 2, 1>(c, lut, o, d, t0, t1, color, opacity, ns);
+    else
+      march_xp<I64, U, LUT_GLOBAL, 2, 0>(c, lut, o, d, t0, t1, color, opacity, ns);
+  } else if (c.dims[0] >= 2)
     march_xp<I64, U, LUT_GLOBAL, SKIP, 1>(c, lut, o, d, t0, t1, color, opacity, ns);
   else
     march_xp<I64, U, LUT_GLOBAL, SKIP, 0>(c, lut, o, d, t0, t1, color, opacity, ns);
