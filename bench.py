@@ -559,7 +559,7 @@ def main():
         traffic = load_traffic("render_spheres10m_1920x1080")
         # HBM bytes of the kernel instance the autotuner picked (both node
         # widths are profiled)
-        inst = f"k_render<1, false, 0, {'true' if tw == 4 else 'false'}>"
+        inst = f"k_render<1, false, 0, {2 if tw == 4 else 0}>"
         tb = [v for k, v in (traffic or {}).get("per_kernel", {}).items() if inst in k]
         roofline = {"bound": "hbm", "achieved": round(achieved, 2), "peak": HBM_PEAK_GBS,
                     "unit": "GB/s", "frac": round(achieved / HBM_PEAK_GBS, 4),

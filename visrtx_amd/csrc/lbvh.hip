@@ -1026,9 +1026,11 @@ __device__ __forceinline__ void refit_list(const vrx_prims &p, const void *leave
 // the top pass.  The span's nodes are listed in index order (ordered
 // compaction of the level bytes); each finds its parent's list slot by a
 // binary search, and the nodes are refit by bottom-up walks with LDS
-// arrival counters, as in pass 1, with the boxes in memory: a child node is
-// a pass-1 node of the previous launch, or a pass-2 node this workgroup
-// wrote before the arrival add that lets its parent go.
+// arrival counters, as in pass 1.  A list that fits (refit_list) keeps its
+// boxes in LDS too and writes its nodes at the end.  A longer one keeps them
+// in memory: a child node is a pass-1 node of the previous launch, or a
+// pass-2 node this workgroup wrote before the arrival add that lets its
+// parent go.
 template <int T>
 __global__ __launch_bounds__(kSpanThreads) void k_refit_span(vrx_prims p, const void *leaves,
     const uint32_t *ids, const uint2 *child, const uint8_t *level, Node *nodes, uint32_t *top,

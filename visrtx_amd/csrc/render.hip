@@ -67,11 +67,12 @@ __global__ __launch_bounds__(kBlock) void k_render(vrx_scene sc, vrx_camera cam,
   render_tile<PT, TWO, KIND, WIDE>(sc, cam, r, f, sd, ovf_cap, scratch);
 }
 
-// The same program held to 80 VGPRs (6 waves per SIMD), for the
-// primitive-specialised AO and directLight programs and two-level raycast:
-// their secondary rays and instance walks are latency-bound, and the extra
-// waves outweigh the registers spilled to scratch (10M spheres: AO 16 spp
-// 13.1 -> 11.9 ms, directLight 4 spp 6.4 -> 5.7 ms; 1M instances +7 %).
+// The same program held to 80 VGPRs (6 waves per SIMD), for two-level raycast
+// and for the primitive-specialised AO and directLight programs that
+// k_render_sampled does not take: their secondary rays and instance walks are
+// latency-bound, and the extra waves outweigh the registers spilled to
+// scratch (BVH2 nodes, 10M spheres: AO 16 spp 13.1 -> 11.9 ms, directLight
+// 4 spp 6.4 -> 5.7 ms; 1M instances +7 %).
 // Single-level raycast (66-88 VGPRs) and the generic kernel (130-150 VGPRs)
 // keep k_render.
 template <int PT, bool TWO, int KIND, int WIDE>
