@@ -514,9 +514,9 @@ __device__ __forceinline__ float jittered_start(const vrx_volume &V, const VolCt
   return t0 + c.step * pcg_float(*jit);
 }
 
-__device__ float march_all(const vrx_scene &sc, v3 o, v3 d, float tlower, float tfar,
-    float inv_rate, v3 &color, float &opacity, uint32_t &obj, uint32_t &inst, uint32_t &ns,
-    bool skip, Pcg *jit = nullptr)
+__device__ __forceinline__ float march_all(const vrx_scene &sc, v3 o, v3 d, float tlower,
+    float tfar, float inv_rate, v3 &color, float &opacity, uint32_t &obj, uint32_t &inst,
+    uint32_t &ns, bool skip, Pcg *jit = nullptr)
 {
   float depth = tfar;
   bool first = true;
@@ -653,8 +653,8 @@ __device__ __forceinline__ float surface_atten(
 // computeAO (gpu/computeAO.h:38-60): n cosine-weighted hemisphere rays from
 // the geometric-normal offset point, four PCG draws each.
 template <int PT, bool TWO, int WIDE>
-__device__ float ao_factor(const vrx_scene &sc, const SurfHit &s, float dist, int n, Pcg &rs,
-    Stack &st, uint32_t &rays)
+__device__ __forceinline__ float ao_factor(const vrx_scene &sc, const SurfHit &s, float dist,
+    int n, Pcg &rs, Stack &st, uint32_t &rays)
 {
   float weights = 0.0f, hits = 0.0f;
   for (int k = 0; k < n; k++) {
@@ -676,8 +676,8 @@ __device__ float ao_factor(const vrx_scene &sc, const SurfHit &s, float dist, in
 // :270-279): every volume the shadow ray crosses on [0, tmax] is marched into
 // one opacity (rayMarchVolume without colour, volumeIntegration.h:64-103),
 // volumes in index order, stopping at 0.99.
-__device__ float volume_atten(const vrx_scene &sc, v3 o, v3 d, float tmax, float inv_rate,
-    bool skip, uint32_t &ns, Pcg *jit = nullptr)
+__device__ __forceinline__ float volume_atten(const vrx_scene &sc, v3 o, v3 d, float tmax,
+    float inv_rate, bool skip, uint32_t &ns, Pcg *jit = nullptr)
 {
   float opacity = 0.0f;
   for (uint32_t i = 0; i < sc.num_volumes && opacity < 0.99f; i++) {
@@ -748,8 +748,8 @@ __device__ __forceinline__ LightSample sample_light(const vrx_light *L, v3 hp)
 // (their nextRay is zero), so the bounce loop ends at once.  Returns the
 // colour and the material opacity.
 template <int PT, bool TWO, int WIDE>
-__device__ float4 shade_direct(const vrx_scene &sc, const vrx_renderer &r, const SurfHit &s,
-    int aos, Pcg &rs, Stack &st, uint32_t &rays, uint32_t &vsamples)
+__device__ __forceinline__ float4 shade_direct(const vrx_scene &sc, const vrx_renderer &r,
+    const SurfHit &s, int aos, Pcg &rs, Stack &st, uint32_t &rays, uint32_t &vsamples)
 {
   const v3 sp = add(s.hp, fmul(s.eps, s.ns));
   const float aof =
