@@ -391,9 +391,11 @@ typedef struct vrx_diffvol {
   int32_t checkpoint;      /* steps between transmittance checkpoints (64) */
   uint32_t max_steps;      /* per ray upper bound (for checkpoint storage) */
   /* optional layout hint: rays are images of image_w x image_h, row-major,
-   * one after another (as vrx_make_rays writes them); the adjoint then gives
-   * each workgroup a 16x16 pixel tile so neighbouring rays share gradient
-   * scatter.  0 = rays in no particular order. */
+   * one after another (as vrx_make_rays writes them); forward and adjoint then
+   * give each wave an 8x8 pixel tile, so that neighbouring rays share cache
+   * lines and gradient scatter.  0 = rays in no particular order.  Images that
+   * do not divide the ray count: the forward takes the rays in no order, the
+   * adjoint refuses them. */
   uint32_t image_w, image_h;
   int32_t adjoint;         /* vrx_adjoint: backward schedule */
 } vrx_diffvol;
@@ -408,9 +410,20 @@ enum vrx_adjoint { VRX_ADJOINT_SUFFIX = 0, VRX_ADJOINT_REPLAY = 1 };
 /* rays: n origins/directions (float3) */
 int vrx_diffvol_forward(const vrx_diffvol *v, uint32_t n, const float *d_org, const float *d_dir,
     float *d_rgba_out, float *d_ckpt, vrx_stream s);
+/* The same forward with work space (16-byte aligned; free for other use once
+ * the stream has passed this call) for a copy of the field as y-pairs, which
+ * many rays repay: vrx_diffvol_workspace_bytes gives its size, 0 where rays
+ * and grid gain nothing by it.  NULL or less than that: vrx_diffvol_forward.
+ * The outputs are the same bits either way. */
+size_t vrx_diffvol_workspace_bytes(const vrx_diffvol *v, uint32_t n);
+int vrx_diffvol_forward_ws(const vrx_diffvol *v, uint32_t n, const float *d_org,
+    const float *d_dir, float *d_rgba_out, float *d_ckpt, void *d_workspace,
+    size_t workspace_bytes, vrx_stream s);
 int vrx_diffvol_backward(const vrx_diffvol *v, uint32_t n, const float *d_org, const float *d_dir,
     const float *d_rgba, const float *d_grad_rgba, const float *d_ckpt,
     float *d_grad_density, float *d_grad_lut, vrx_stream s);
+/* floats of d_ckpt: n times a number of max_steps and checkpoint alone, so a
+ * buffer for n rays serves fewer rays and every grid of no more steps */
 size_t vrx_diffvol_ckpt_floats(const vrx_diffvol *v, uint32_t n);
 /* pinhole rays for a set of views: cams[nviews], w x h each (row 0 = bottom) */
 int vrx_make_rays(const vrx_camera *cams, uint32_t nviews, uint32_t w, uint32_t h,

@@ -2,10 +2,13 @@
 y-pair gathers that 65,536 rays and more take.  All sample the same positions
 in the same order, so a ray's colour and opacity are bit-identical; the
 gradients of a loss over all rays differ by the order of their 32-bit sums."""
+import ctypes as C
+
 import numpy as np
 import pytest
 import torch
 
+from visrtx_amd import _native as N
 from visrtx_amd import diffvol as D
 from visrtx_amd import scenes as S
 
@@ -54,3 +57,34 @@ def test_gradients_of_many_rays(require_gpu):
         got.append((d.grad, l.grad))
     for a, b in zip(*got):
         assert float((a - b).norm() / b.norm()) < 2e-5
+
+
+@pytest.mark.parametrize("dims", [(64, 64, 64), (17, 9, 33)])
+def test_work_space_does_not_change_the_rays(require_gpu, dims):
+    """With work space, with too little of it and through the entry point that
+    takes none; the checkpoints hold exactly what the size query says."""
+    dens, lut, org, dirs, spec = _setup(dims, (64, 64))
+    s = D.GridSpec(**spec, image=(64, 64))
+    v, n, L = s.struct(dens, lut), len(org), N.hip()
+    floats = L.vrx_diffvol_ckpt_floats(C.byref(v), n)
+    need = L.vrx_diffvol_workspace_bytes(C.byref(v), n)
+    assert need == 8 * dens.numel()
+    ws = torch.full((need + 256,), 7, device="cuda", dtype=torch.uint8)
+    out = []
+    for form, size in (("none", 0), ("short", need - 1), ("whole", need)):
+        print(f"[forward] {dims} work space {form}", flush=True)
+        rgba = torch.empty((n, 4), device="cuda")
+        ck = torch.full((floats + 64,), -7.0, device="cuda")
+        args = (C.byref(v), n, org.data_ptr(), dirs.data_ptr(), rgba.data_ptr(), ck.data_ptr())
+        if form == "none":
+            N.check(L.vrx_diffvol_forward(*args, None))
+        else:
+            N.check(L.vrx_diffvol_forward_ws(*args, ws.data_ptr(), size, None))
+        torch.cuda.synchronize()
+        assert (ck[floats:] == -7.0).all() and (ws[need:] == 7).all()
+        out.append((rgba, ck.view(torch.int32)))
+    assert (ws[:need] != 7).any()
+    assert L.vrx_diffvol_forward_ws(*args, ws.data_ptr() + 4, need, None) == -2
+    # slots that a ray does not use keep their fill
+    for rgba, ck in out[1:]:
+        assert torch.equal(rgba, out[0][0]) and torch.equal(ck, out[0][1])

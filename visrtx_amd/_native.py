@@ -191,6 +191,8 @@ def hip() -> C.CDLL:
             "vrx_tlas_query_sizes": (i32, [u32, vp]),
             "vrx_tlas_build": (i32, [vp, vp, vp, sz, vp]),
             "vrx_diffvol_forward": (i32, [vp, u32, vp, vp, vp, vp, vp]),
+            "vrx_diffvol_forward_ws": (i32, [vp, u32, vp, vp, vp, vp, vp, sz, vp]),
+            "vrx_diffvol_workspace_bytes": (sz, [vp, u32]),
             "vrx_diffvol_backward": (i32, [vp, u32, vp, vp, vp, vp, vp, vp, vp, vp]),
             "vrx_diffvol_ckpt_floats": (sz, [vp, u32]),
             "vrx_make_rays": (i32, [vp, u32, u32, u32, vp, vp, vp]),

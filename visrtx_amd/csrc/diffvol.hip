@@ -808,17 +808,9 @@ __global__ void k_make_rays(CamBlock cams, uint32_t first_view, uint32_t nviews,
   gst(dir, 3 * i + 2, dd.z);
 }
 
-// floats of the march's own part of d_ckpt: count, final T, T every ck steps,
-// then the FP64 totals (8 words)
-static size_t march_floats(const vrx_diffvol *v, uint32_t n)
-{
-  const int ck = v->checkpoint > 0 ? v->checkpoint : 64;
-  return (size_t)(2 + (v->max_steps + ck - 1) / ck + 8) * n;
-}
-
-// The forward copies the density to y-pairs behind the checkpoints where its
-// rays repay the copy: it moves 12 B per voxel (3.5 ps a voxel and a launch),
-// and the gathers save 94 ps per ray (at some 45 samples).
+// The forward copies the density to y-pairs where its rays repay the copy: it
+// moves 12 B per voxel (3.5 ps a voxel and a launch), and the gathers save
+// 94 ps per ray (at some 45 samples).
 static bool use_pairs(const vrx_diffvol *v, uint32_t n)
 {
   const uint64_t vox = (uint64_t)v->dims[0] * v->dims[1] * v->dims[2];
@@ -845,14 +837,19 @@ size_t vrx_diffvol_ckpt_floats(const vrx_diffvol *v, uint32_t n)
 {
   if (!v)
     return 0;
-  size_t f = march_floats(v, n);
-  if (use_pairs(v, n))
-    f = ((f + 3) & ~size_t(3)) + 2 * (size_t)v->dims[0] * v->dims[1] * v->dims[2];
-  return f;
+  int ck = v->checkpoint > 0 ? v->checkpoint : 64;
+  // count, final T, T every ck steps, then the FP64 totals (8 words)
+  return (size_t)(2 + (v->max_steps + ck - 1) / ck + 8) * n;
 }
 
-int vrx_diffvol_forward(const vrx_diffvol *v, uint32_t n, const float *d_org, const float *d_dir,
-    float *d_rgba_out, float *d_ckpt, vrx_stream s)
+size_t vrx_diffvol_workspace_bytes(const vrx_diffvol *v, uint32_t n)
+{
+  return v && use_pairs(v, n) ? (size_t)v->dims[0] * v->dims[1] * v->dims[2] * 8 : 0;
+}
+
+int vrx_diffvol_forward_ws(const vrx_diffvol *v, uint32_t n, const float *d_org,
+    const float *d_dir, float *d_rgba_out, float *d_ckpt, void *d_workspace,
+    size_t workspace_bytes, vrx_stream s)
 {
   int st = check_dv(v);
   if (st)
@@ -860,14 +857,16 @@ int vrx_diffvol_forward(const vrx_diffvol *v, uint32_t n, const float *d_org, co
   if (n == 0)
     return VRX_OK;
   VRX_ARG(d_org && d_dir && d_rgba_out && d_ckpt, "ray/output buffers");
+  VRX_ARG(((uintptr_t)d_workspace & 15u) == 0, "workspace alignment");
   DvCtx c = make_ctx(*v);
   const size_t per = (size_t)c.img_w * c.img_h;
   if (per == 0 || n % per != 0)
     c.img_w = 0; // whole images only; otherwise rays in no particular order
   const uint32_t nb = c.img_w > 0 ? (uint32_t)(n / per) * c.tiles_per_img
                                   : (n + kDvBlock - 1) / kDvBlock;
-  if (use_pairs(v, n)) {
-    float *pairs = d_ckpt + ((march_floats(v, n) + 3) & ~size_t(3));
+  const size_t need = vrx_diffvol_workspace_bytes(v, n);
+  if (need && d_workspace && workspace_bytes >= need) {
+    float *pairs = (float *)d_workspace;
     vrx_volume f;
     memset(&f, 0, sizeof(f));
     f.d_data = v->d_density;
@@ -882,6 +881,12 @@ int vrx_diffvol_forward(const vrx_diffvol *v, uint32_t n, const float *d_org, co
   }
   VRX_LAUNCH_CHECK();
   return VRX_OK;
+}
+
+int vrx_diffvol_forward(const vrx_diffvol *v, uint32_t n, const float *d_org, const float *d_dir,
+    float *d_rgba_out, float *d_ckpt, vrx_stream s)
+{
+  return vrx_diffvol_forward_ws(v, n, d_org, d_dir, d_rgba_out, d_ckpt, nullptr, 0, s);
 }
 
 int vrx_diffvol_backward(const vrx_diffvol *v, uint32_t n, const float *d_org, const float *d_dir,

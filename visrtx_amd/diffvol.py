@@ -88,8 +88,12 @@ class VolumeIntegral(torch.autograd.Function):
         rgba = torch.empty((n, 4), device=org.device, dtype=torch.float32)
         ck = torch.empty(L.vrx_diffvol_ckpt_floats(C.byref(v), n), device=org.device,
                          dtype=torch.float32)
-        N.check(L.vrx_diffvol_forward(C.byref(v), n, org.data_ptr(), dirs.data_ptr(),
-                                      rgba.data_ptr(), ck.data_ptr(), _stream()),
+        # work space of this call alone, on its stream
+        nb = L.vrx_diffvol_workspace_bytes(C.byref(v), n)
+        ws = torch.empty(nb, device=org.device, dtype=torch.uint8) if nb else None
+        N.check(L.vrx_diffvol_forward_ws(C.byref(v), n, org.data_ptr(), dirs.data_ptr(),
+                                         rgba.data_ptr(), ck.data_ptr(),
+                                         ws.data_ptr() if nb else None, nb, _stream()),
                 "vrx_diffvol_forward")
         ctx.save_for_backward(density, lut, org, dirs, rgba, ck)
         ctx.spec = spec
