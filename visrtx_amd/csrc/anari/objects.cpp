@@ -1586,6 +1586,9 @@ int World::rebuild()
   vrx_event_destroy(e1);
   memcpy(bounds, wb, sizeof(bounds));
   hostGeoms = std::move(hg);
+  numPrims = 0;
+  for (const vrx_geom &g : hostGeoms)
+    numPrims += g.n;
   hostGeomOf = std::move(geomOf);
   sceneDirty = false;
   builtAt = dev->tick();
@@ -1898,25 +1901,54 @@ bool Frame::ready()
 // one-level scenes with one primitive type)
 constexpr int kLongRaySteps = 32;
 
+// A launch chosen on one state of a world that is rebuilt can be several times
+// slower than another on a later state (10M spheres: 1.87 ms with the long-ray
+// pass, 0.43 without), so the frames of rebuilt worlds are compared with the
+// time that won.  Two of eight by more than 1.5x to either side (a lighter
+// scene can hide a bad launch): measure again.  If that happens three times
+// within kTuneSoon frames of the choice, the frames alternate between states
+// that no choice fits, and the first candidate, without the long-ray pass,
+// stays.
+constexpr float kTuneBand = 1.5f;
+constexpr uint32_t kTuneSoon = 32;
+
+bool Frame::rebuiltOff()
+{
+  float ms = 0.0f;
+  if (tune.best < 0 || tune.n < 2 || tune.settled || tune.lastBuild == tune.chosenBuild
+      || vrx_event_elapsed_ms(evStart, evEnd, &ms) != 0)
+    return false;
+  const float won = tune.ms[tune.best];
+  const bool off = ms > kTuneBand * won || won > kTuneBand * ms;
+  tune.off = (uint8_t)(tune.off << 1 | (off ? 1 : 0));
+  tune.watched++;
+  return __builtin_popcount(tune.off) >= 2;
+}
+
 void Frame::pickLaunch(vrx_renderer &rr)
 {
-  // a rebuilt world of the same shape (a mesh deformed every frame) keeps what
-  // its frames have measured: starting over with every rebuild, it rendered
-  // with the first candidate for ever (131k deforming triangles at 1024x768:
-  // 146 us a frame's kernel instead of 105 with the long-ray pass)
-  uint64_t prims = 0;
-  for (const vrx_geom &g : world->hostGeoms)
-    prims += g.n;
-  uint64_t shape = 0;
-  for (; prims; prims >>= 1)
-    shape++;
-  shape = (shape << 40) ^ ((uint64_t)world->scene.num_entries << 8)
-      ^ ((uint64_t)world->scene.num_volumes << 4) ^ (uint64_t)(world->scene.single_type + 1);
-  uint64_t key = (uint64_t)(uintptr_t)world ^ (shape << 20) ^ (uint64_t)(uintptr_t)renderer
-      ^ (renderer->lastFinalized << 40) ^ ((uint64_t)size[0] << 8) ^ ((uint64_t)size[1] << 28);
-  if (key != tune.key) {
+  // A rebuilt world keeps what its frames have measured: starting over with
+  // every rebuild, it rendered with the first candidate for ever (131k
+  // deforming triangles at 1024x768: 146 us a frame's kernel instead of 105
+  // with the long-ray pass).
+  Tune::Key key;
+  key.world = world;
+  key.renderer = renderer;
+  key.finalized = renderer->lastFinalized;
+  key.width = size[0];
+  key.height = size[1];
+  key.entries = world->scene.num_entries;
+  key.volumes = world->scene.num_volumes;
+  key.type = world->scene.single_type;
+  for (uint64_t p = world->numPrims; p; p >>= 1)
+    key.primBits++;
+  const bool known = key == tune.key;
+  const bool again = known && rebuiltOff();
+  if (!known || again) {
+    const int hasty = again && tune.watched <= kTuneSoon ? tune.hasty + 1 : 0;
     tune = Tune{};
     tune.key = key;
+    tune.hasty = hasty;
     // the first frame also pays for cold caches and page tables, so its stack
     // depth is tried again last.  BVH2 nodes are not tried: the packed 4-wide
     // nodes are faster on every scene measured (10M spheres 0.45 against
@@ -1939,6 +1971,10 @@ void Frame::pickLaunch(vrx_renderer &rr)
       tune.defer[tune.n] = tune.deferPending ? 0 : rr.defer_steps;
       tune.n++;
     }
+    if (hasty >= 3) {
+      tune.settled = true;
+      tune.best = 0;
+    }
   } else if (tune.best < 0 && tune.last >= 0) {
     // the previous render used candidate `last`; wait() has made its events
     // complete
@@ -1959,9 +1995,11 @@ void Frame::pickLaunch(vrx_renderer &rr)
         tune.n++;
       } else {
         tune.best = b;
+        tune.chosenBuild = tune.lastBuild;
       }
     }
   }
+  tune.lastBuild = world->builtAt;
   const int use = tune.best >= 0 ? tune.best : tune.next;
   if (tune.best < 0)
     tune.next++;

@@ -295,6 +295,7 @@ struct World : Object {
   float lastBuildMs{0.0f}, lastWideMs{0.0f};
   // host copies of the scene tables (for re-upload when 4-wide nodes appear)
   std::vector<vrx_geom> hostGeoms;
+  uint64_t numPrims{0}; // of hostGeoms
   std::vector<Geometry *> hostGeomOf;
   int rebuild();
   int ensureWide(); // 4-wide nodes for every BLAS and the TLAS; sets scene.wide
@@ -354,17 +355,41 @@ struct Frame : Object {
   vrx_event evDone{nullptr}; // after the result read-backs that follow evEnd
   bool rendered{false};
   bool stackReported{false};
-  // Online launch autotuning: the first frames of a (world, renderer, size)
-  // configuration each use one candidate (node width x LDS stack depth), timed
-  // by the frame's events; then the fastest is kept.  Every candidate gives
+  // Online launch autotuning: the first frames of a configuration each use one
+  // candidate (node width x LDS stack depth, then the long-ray pass), timed by
+  // the frame's events; then the fastest is kept.  Every candidate gives
   // bit-identical channels, so tuning only changes the time.
   struct Tune {
-    uint64_t key{0};
+    // what the measurements belong to.  A world that is rebuilt with as many
+    // entries and volumes, the same primitive type and a like number of
+    // primitives (a mesh deformed every frame) keeps them.
+    struct Key {
+      const World *world{nullptr};
+      const Renderer *renderer{nullptr};
+      uint64_t finalized{0}; // the renderer's last commit
+      uint32_t width{0}, height{0};
+      uint32_t entries{0}, volumes{0};
+      int32_t type{0};
+      uint32_t primBits{0}; // bits of the primitive count
+      bool operator==(const Key &k) const
+      {
+        return world == k.world && renderer == k.renderer && finalized == k.finalized
+            && width == k.width && height == k.height && entries == k.entries
+            && volumes == k.volumes && type == k.type && primBits == k.primBits;
+      }
+    } key;
     int n{0}, next{0}, best{-1}, last{-1};
     bool deferPending{false}; // the long-ray candidate is still to be added
     int width[8]{}, sd[8]{}, defer[8]{};
     float ms[8]{};
+    // frames of worlds rebuilt since the choice are watched (rebuiltOff())
+    uint64_t chosenBuild{0}, lastBuild{0}; // the world's build at the choice, of the last frame
+    uint32_t watched{0};                   // frames watched
+    uint8_t off{0};                        // the last eight of them, bit set: off
+    int hasty{0};                          // choices in a row that soon went off
+    bool settled{false};                   // no more choices for this key
   } tune;
+  bool rebuiltOff();
   void pickLaunch(vrx_renderer &rr);
   // completion callbacks: each render with a callback posts one job; the
   // device's callback thread runs it and advances `sync`
