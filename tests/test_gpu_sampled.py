@@ -4,6 +4,7 @@ and sums, so opaque frames are bit-identical.  Translucent ones differ by the
 order in which a shadow ray's surfaces are added, a few 1e-7 per surface; 1e-5
 allows for the layers.  Sizes: none to more secondary rays per hit than the
 queue holds for one pixel (6), frames of partial tiles, accumulation."""
+import ctypes as C
 import math
 
 import numpy as np
@@ -11,7 +12,9 @@ import pytest
 
 from tests.test_gpu_packed import _prims
 from tests.test_gpu_render import render_gpu
+from visrtx_amd import _native as N
 from visrtx_amd import anari as A
+from visrtx_amd import batch as B
 from visrtx_amd import scenes as S
 
 pytestmark = pytest.mark.gpu
@@ -110,3 +113,26 @@ def test_opacity_above_one(require_gpu):
     sc = _scene("sphere", 300, LIGHTS[:1], 1.5)
     assert math.isfinite(sc.geoms[0].opacity)
     _compare(sc, 32, 32, "directLight", exact=False, pixelSamples=2, ambientSamples=1)
+
+
+def test_queues_are_those_of_the_resident_waves(require_gpu):
+    """The frame scratch grows by a queue (16 words a ray, six rays a lane) for
+    each wave that can be resident, 20 per compute unit at the kernel's
+    registers, or for each wave of a small frame."""
+    dev = A.Device()
+    s = S.build_anari(dev, _scene("sphere", 100))
+    scene = B.scene_of(dev, s.world, wide=True)
+    got = {}
+    for kind in ("raycast", "ao"):
+        r = B.renderer_of(dev, S.make_renderer(dev, s, kind, nodeWidth=4))
+        r.defer_steps = 0
+        got[kind] = {wh: N.hip().vrx_render_scratch_bytes(C.byref(scene), C.byref(r), *wh)
+                     for wh in ((1920, 1080), (64, 48), (1, 1))}
+    s.release()
+    dev.close()
+    cus, queue = C.c_int(), 16 * 4 * 6 * 64
+    N.check(N.hip().vrx_device_info(0, None, 0, C.byref(cus), None))
+    extra = {wh: got["ao"][wh] - got["raycast"][wh] for wh in got["ao"]}
+    print(f"[sampled] queues {extra}, {cus.value} compute units", flush=True)
+    for wh, blocks in (((1920, 1080), 5 * cus.value), ((64, 48), 12), ((1, 1), 1)):
+        assert 0 < extra[wh] <= 4 * blocks * queue

@@ -764,12 +764,17 @@ static size_t long_queue_offset(uint32_t width, uint32_t height, uint32_t cap)
   return 256 + tiles * kBlock * (size_t)cap * 4;
 }
 
-// Byte offset of the ray queues in the frame scratch (after the stack-spill
-// area) and their bytes: one queue per wave of the largest resident grid.
+// The ray queues of k_render_sampled, after the rest of the frame scratch: one
+// per wave of its largest grid.  The kernel's 96 registers let 5 of its blocks
+// of four waves reside on a compute unit, so the grid is no larger than that
+// (118 MB of queues on 256 compute units; a frame of under 1280 tiles of 16x16
+// pixels has fewer blocks).
+constexpr uint32_t kSampledBlocksPerCu = 5;
+
 static uint32_t sampled_max_blocks(uint32_t width, uint32_t height)
 {
   const uint64_t tiles = (uint64_t)((width + kTile - 1) / kTile) * ((height + kTile - 1) / kTile);
-  return (uint32_t)std::min<uint64_t>(tiles, (uint64_t)device_cus() * 8);
+  return (uint32_t)std::min<uint64_t>(tiles, (uint64_t)device_cus() * kSampledBlocksPerCu);
 }
 
 static size_t sampled_queue_bytes(uint32_t width, uint32_t height)

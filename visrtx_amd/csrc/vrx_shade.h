@@ -992,12 +992,12 @@ __device__ __forceinline__ bool trace_group(const vrx_scene &sc, v3 wo, v3 wd, f
 // finish.  The results are then summed per pixel in render_pixel()'s order,
 // and the random draws are the same, so the pixels are the same.
 // Measured against render_pixel() on the same nodes: AO 16 spp on 10M spheres
-// 11.1 -> 10.8 ms with 1 AO ray per hit (closest walks are half of the steps
+// 11.1 -> 10.4 ms with 1 AO ray per hit (closest walks are half of the steps
 // there), 4 spp with 2 lights and 1 AO ray on 1M spheres 3.84 -> 3.10 ms;
 // 3 slots instead of 6 are 4 % slower, 12 as fast; workgroup-wide tiles 6 %
 // slower than a tile per wave (its waves wait for one another).
 constexpr int kQueueSlots = 6;    // rays per pixel and round
-constexpr int kQueueWords = 12;   // origin, direction, weight (3), tmax, result, unused
+constexpr int kQueueWords = 11;   // origin, direction, weight (3), tmax, result
 constexpr int kSampleWords = 4;   // surface colour and opacity
 constexpr uint32_t kQueueFloats = (kQueueSlots * (kQueueWords + kSampleWords)) * 64; // per wave
 
