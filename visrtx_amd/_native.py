@@ -72,6 +72,23 @@ class vrx_bvh_header(C.Structure):
                 ("n", C.c_uint32), ("type", C.c_int32), ("pad", C.c_uint32 * 6)]
 
 
+class vrx_geom(C.Structure):
+    _fields_ = [("type", C.c_int32), ("n", C.c_uint32), ("bvh", vrx_bvh),
+                ("d_position", C.c_void_p), ("d_index", C.c_void_p), ("d_radius", C.c_void_p),
+                ("global_radius", C.c_float), ("d_primitive_id", C.c_void_p),
+                ("d_vertex_normal", C.c_void_p), ("caps", C.c_int32),
+                ("cull_backfaces", C.c_int32), ("color", f3), ("opacity", C.c_float),
+                ("surface_id", C.c_uint32), ("pad", C.c_uint32)]
+
+
+class vrx_frame(C.Structure):
+    _fields_ = [("width", C.c_uint32), ("height", C.c_uint32), ("color_format", C.c_int32),
+                ("frame_id", C.c_uint32), ("d_accum", C.c_void_p), ("d_color_f32", C.c_void_p),
+                ("d_color_u32", C.c_void_p), ("d_depth", C.c_void_p), ("d_prim_id", C.c_void_p),
+                ("d_obj_id", C.c_void_p), ("d_inst_id", C.c_void_p), ("d_scratch", C.c_void_p),
+                ("scratch_bytes", C.c_size_t), ("d_counters", C.c_void_p)]
+
+
 class vrx_camera(C.Structure):
     _fields_ = [("pos", f3), ("d00", f3), ("du", f3), ("dv", f3), ("region", f4)]
 
