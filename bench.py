@@ -553,20 +553,23 @@ def main():
         extra["tuned_launch"] = {"node_width": tw, "stack_lds": tsd}
         extra["primary_kernel_mrays_s"] = round(rays / (kern_ms / 1000) / 1e6, 2)
         c2 = counts["spheres10m_1920x1080"]
+        # bytes of the oracle's BVH2 walk; the caches serve most of what a
+        # launch reads, so they say nothing about HBM
         bytes_per_ray = 32 + 16 + 64 * c2["nodes_per_ray"] + 16 * c2["prims_per_ray"]
-        alg_bytes = rays * bytes_per_ray
-        achieved = alg_bytes / (kern_ms / 1000) / 1e9
         traffic = load_traffic("render_spheres10m_1920x1080")
-        # HBM bytes of the kernel instance the autotuner picked (both node
-        # widths are profiled)
+        # profiled HBM bytes of the kernel instance the autotuner picked (both
+        # node widths are profiled) over this run's kernel time
         inst = f"k_render<1, false, 0, {2 if tw == 4 else 0}>"
         tb = [v for k, v in (traffic or {}).get("per_kernel", {}).items() if inst in k]
-        roofline = {"bound": "hbm", "achieved": round(achieved, 2), "peak": HBM_PEAK_GBS,
-                    "unit": "GB/s", "frac": round(achieved / HBM_PEAK_GBS, 4),
+        achieved = tb[0] / (kern_ms / 1000) / 1e9 if tb else None
+        roofline = {"bound": "hbm", "limiter": "VALU and the L1 data path",
+                    "achieved": round(achieved, 2) if tb else None, "peak": HBM_PEAK_GBS,
+                    "unit": "GB/s", "frac": round(achieved / HBM_PEAK_GBS, 4) if tb else None,
                     "traffic": tb[0] if tb else None,
                     "kernel": f"k_render<sphere,single-level,raycast,{tw}-wide nodes>",
                     "stack_lds": tsd,
-                    "algorithmic_bytes_per_ray": round(bytes_per_ray, 2),
+                    "bvh2_walk_bytes_per_ray": round(bytes_per_ray, 2),
+                    "bvh2_walk_gbs": round(rays * bytes_per_ray / (kern_ms / 1000) / 1e9, 1),
                     "avg_kernel_ms": round(kern_ms, 4)}
         extra["widen_ms_10m_spheres"] = round(
             1000.0 * dev.get_property(work.s.world, "bvhWidenDuration", A.FLOAT32), 3)
@@ -658,14 +661,12 @@ def main():
         dev.commit(hf.r)
         _, d13 = hf.timed(20, 3)
         extra["heightfield_kernel_ms_no_long_ray_pass"] = round(statistics.mean(d13) * 1000, 4)
-        # roofline of the tuned kernel: algorithmic traversal bytes per ray
-        # (ray in, hit out, 64-B nodes and 48-B triangles the oracle visits)
+        # bytes of the oracle's BVH2 walk (ray in, hit out, 64-B nodes, 48-B
+        # triangles), mostly served by the caches
         c1 = counts["heightfield_1024x768"]
         bpr1 = 32 + 16 + 64 * c1["nodes_per_ray"] + 48 * c1["prims_per_ray"]
         gbs1 = 1024 * 768 * bpr1 / (extra["heightfield_kernel_ms"] / 1000) / 1e9
-        extra["heightfield_roofline"] = {"bound": "hbm", "algorithmic_bytes_per_ray": round(bpr1, 2),
-                                         "achieved_gbs": round(gbs1, 1),
-                                         "frac": round(gbs1 / HBM_PEAK_GBS, 4)}
+        extra["heightfield_bvh2_walk"] = {"bytes_per_ray": round(bpr1, 2), "gbs": round(gbs1, 1)}
         log(f"heightfield: {sps * 1000:.3f} ms/step -> {extra['heightfield_mrays_s']} Mrays/s")
         hf.release()
 
@@ -722,14 +723,13 @@ def main():
     if "batched" in sec:
         log("batched 64 views")
         bt = bench_batched(dev)
-        # roofline of the graph-replayed launch: traversal bytes per ray from
-        # the oracle's counts on views 0 and 37 (BLAS nodes and triangles)
+        # bytes of the oracle's BVH2 walk on views 0 and 37 (BLAS nodes and
+        # triangles) over the graph-replayed launch
         c4 = counts["batched_views0_37_512"]
         bpr4 = 32 + 16 + 64 * c4["nodes_per_ray"] + 48 * c4["prims_per_ray"]
         gbs4 = bt["rays"] * bpr4 / (bt["batched_graph_event_ms"] / 1000) / 1e9
-        bt["roofline"] = {"bound": "hbm", "algorithmic_bytes_per_ray": round(bpr4, 1),
-                          "achieved_gbs": round(gbs4, 1), "frac": round(gbs4 / HBM_PEAK_GBS, 4),
-                          "counts": "oracle, views 0 and 37"}
+        bt["bvh2_walk"] = {"bytes_per_ray": round(bpr4, 1), "gbs": round(gbs4, 1),
+                           "counts": "oracle, views 0 and 37"}
         extra["batched_64x512"] = bt
         log(f"batched: plain {bt['plain_ms']} ms, graph {bt['batched_graph_ms']} ms "
             f"-> {bt['speedup_vs_plain']}x ({bt['batched_mrays_s']} Mrays/s)")

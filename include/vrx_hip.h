@@ -131,7 +131,9 @@ size_t vrx_bvh_wide_bytes(uint32_t n);
 int vrx_bvh_widen(const vrx_bvh *bvh, uint32_t n, vrx_stream s);
 /* The same 4-wide tree in 64-byte records: child boxes as 8-bit steps on a
  * grid over the record's box, rounded outwards; the traversal checks a hit
- * against its exact leaf box, so frames do not depend on the node format.
+ * against its exact leaf box, so frames do not depend on the node format (but
+ * for the order in which translucent surfaces are added along shadow and AO
+ * rays, a few 1e-7).
  * Writes bvh->d_wide, which must hold vrx_bvh_packed_bytes(type, n); type is
  * the primitive type of the build.  The instance level (VRX_BOX) is packed by
  * vrx_tlas_pack, which also writes a 128-byte record per instance. */
