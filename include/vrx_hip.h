@@ -393,11 +393,9 @@ typedef struct vrx_diffvol {
   int32_t checkpoint;      /* steps between transmittance checkpoints (64) */
   uint32_t max_steps;      /* per ray upper bound (for checkpoint storage) */
   /* optional layout hint: rays are images of image_w x image_h, row-major,
-   * one after another (as vrx_make_rays writes them); forward and adjoint then
-   * give each wave an 8x8 pixel tile, so that neighbouring rays share cache
-   * lines and gradient scatter.  0 = rays in no particular order.  Images that
-   * do not divide the ray count: the forward takes the rays in no order, the
-   * adjoint refuses them. */
+   * one after another (as vrx_make_rays writes them); the adjoint then gives
+   * each wave an 8x8 pixel tile so neighbouring rays share gradient scatter.
+   * 0 = rays in no particular order. */
   uint32_t image_w, image_h;
   int32_t adjoint;         /* vrx_adjoint: backward schedule */
 } vrx_diffvol;

@@ -204,11 +204,12 @@ __device__ __forceinline__ float dv_sample_pairs(const DvCtx &c, const float *pa
 }
 
 // The forward.  It is bound by its gathers' path through L1 (TA 80 % busy,
-// VALU 55 %): a wave per 8x8 pixel tile instead of a row of 64, and a counter
-// instead of a division per sample for the checkpoints, took 128^3, 32 views of
-// 256x256 from 534 to 490 us; the y-pair gathers (PAIRS) to 304, and 8 for the
-// copy.  Gathering two or four samples ahead is no faster (489 and 502 us
-// without pairs).
+// VALU 55 %).  The y-pair gathers (PAIRS) take 128^3, 32 views of 256x256 from
+// 465 to 303 us, 8 of them for the copy; a counter instead of a division per
+// sample finds the checkpoints.  A wave takes 64 consecutive rays: 8x8 pixel
+// tiles of an image are slower (321 us there; without pairs 485; 64^3, 3 views
+// of 501x501: 91 us in rows, 138 in tiles), and gathering two or four samples
+// ahead is no faster.
 template <bool PAIRS>
 __global__ __launch_bounds__(kDvBlock) void k_diffvol_fwd(DvCtx c, const float *lut_g, uint32_t n,
     const float *org, const float *dir, float *rgba, float *ckpt, const float *pairs)
@@ -216,20 +217,7 @@ __global__ __launch_bounds__(kDvBlock) void k_diffvol_fwd(DvCtx c, const float *
   __shared__ float4 s_lut[256];
   s_lut[threadIdx.x] = gld((const float4 *)lut_g, threadIdx.x);
   __syncthreads();
-  uint32_t r;
-  if (c.img_w > 0) {
-    // a wave per 8x8 pixel tile: its samples share more cache lines than a row's
-    const uint32_t img = blockIdx.x / c.tiles_per_img, tile = blockIdx.x - img * c.tiles_per_img;
-    const uint32_t ty = tile / c.tiles_x, tx = tile - ty * c.tiles_x;
-    const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
-    const uint32_t x = tx * 16 + (wave & 1u) * 8 + (lane & 7u);
-    const uint32_t y = ty * 16 + (wave >> 1) * 8 + (lane >> 3);
-    if (x >= c.img_w || y >= c.img_h)
-      return;
-    r = (img * c.img_h + y) * c.img_w + x;
-  } else {
-    r = blockIdx.x * kDvBlock + threadIdx.x;
-  }
+  const uint32_t r = blockIdx.x * kDvBlock + threadIdx.x;
   if (r >= n)
     return;
   const v3 o = gld3(org, r), d = gld3(dir, r);
@@ -808,13 +796,21 @@ __global__ void k_make_rays(CamBlock cams, uint32_t first_view, uint32_t nviews,
   gst(dir, 3 * i + 2, dd.z);
 }
 
-// The forward copies the density to y-pairs where its rays repay the copy: it
-// moves 12 B per voxel (3.5 ps a voxel and a launch), and the gathers save
-// 94 ps per ray (at some 45 samples).
+// The forward copies the density to y-pairs where its rays repay the copy: one
+// ray per 8 voxels (a voxel's copy takes 3.5 ps, the gathers save 30 to 500 ps
+// a ray), and 36M samples over rays that cross the longest side.  With fewer
+// the launch is bound by its latency and the copy only adds to it.  Rays x
+// grid, without and with pairs: 131k x 64^3 41 and 50 us, 131k x 128^3 61 and
+// 71, 262k x 64^3 57 and 59, 753k x 17^3 44 and 46; 262k x 128^3 109 and 81,
+// 524k x 64^3 102 and 88, 524k x 40^3 83 and 77; 262k x 384^3 326 and 404.
 static bool use_pairs(const vrx_diffvol *v, uint32_t n)
 {
   const uint64_t vox = (uint64_t)v->dims[0] * v->dims[1] * v->dims[2];
-  return vox < (1ull << 29) && n >= (1u << 16) && (uint64_t)n * 8 >= vox;
+  float side = 0.0f;
+  for (int k = 0; k < 3; k++)
+    side = std::max(side, ((float)v->dims[k] - 1.0f) * v->spacing[k]);
+  return vox < (1ull << 29) && (uint64_t)n * 8 >= vox
+      && (double)n * (double)(side / v->step) >= 36e6;
 }
 
 static int check_dv(const vrx_diffvol *v)
@@ -859,11 +855,7 @@ int vrx_diffvol_forward_ws(const vrx_diffvol *v, uint32_t n, const float *d_org,
   VRX_ARG(d_org && d_dir && d_rgba_out && d_ckpt, "ray/output buffers");
   VRX_ARG(((uintptr_t)d_workspace & 15u) == 0, "workspace alignment");
   DvCtx c = make_ctx(*v);
-  const size_t per = (size_t)c.img_w * c.img_h;
-  if (per == 0 || n % per != 0)
-    c.img_w = 0; // whole images only; otherwise rays in no particular order
-  const uint32_t nb = c.img_w > 0 ? (uint32_t)(n / per) * c.tiles_per_img
-                                  : (n + kDvBlock - 1) / kDvBlock;
+  const uint32_t nb = (n + kDvBlock - 1) / kDvBlock;
   const size_t need = vrx_diffvol_workspace_bytes(v, n);
   if (need && d_workspace && workspace_bytes >= need) {
     float *pairs = (float *)d_workspace;
