@@ -18,6 +18,8 @@ from tests.devmem import DeviceBuffer
 from tests.test_gpu_render import render_gpu
 from tests.test_oracle_majorants import grid_reference as _grid_reference
 from visrtx_amd import _native as N
+from visrtx_amd import anari as A
+from visrtx_amd import batch as B
 from visrtx_amd import scenes as S
 
 pytestmark = pytest.mark.gpu
@@ -210,3 +212,51 @@ def test_skipping_march_unroll_depths_give_one_frame(require_gpu):
         assert not f["errors"], f["errors"]
         for ch in ("color", "depth", "primitiveId", "objectId", "instanceId"):
             np.testing.assert_array_equal(f[ch], frames[0][ch], err_msg=ch)
+
+
+def test_distances_come_with_the_second_frame_of_a_build(require_gpu):
+    """A world that is rebuilt for every frame does not pay for the grid's
+    distances: the first frame of a build walks the majorants alone, which
+    takes some 10 % longer here, and the next ones the distances.  All give
+    the frame without skipping, and a scene handed out has the distances."""
+    w, h = 1920, 1080
+    sc, cam = S.sparse_volume_workload(256, width=w, height=h)
+    dev = A.Device()
+    s = S.build_anari(dev, sc)
+    c = S.make_camera(dev, s, cam)
+    frames = [S.make_frame(dev, s, s.world, c,
+                           S.make_renderer(dev, s, "raycast", volumeSamplingRate=1.0,
+                                           emptySpaceSkipping=skip), w, h)
+              for skip in (True, False)]
+
+    def render(f):
+        dev.commit(c)
+        dev.render(f)
+        dev.ready(f)
+        return dev.get_property(f, "duration", A.FLOAT32) * 1e6
+
+    render(frames[1])
+    want = [dev.map_frame(frames[1], "channel." + ch)[0] for ch in ("color", "depth", "objectId")]
+    us = [[], [], []]
+    for i in range(16):
+        dev.commit(s.world)
+        for t in us:
+            t.append(render(frames[0]))
+            if i < 2:
+                for ch, x in zip(("color", "depth", "objectId"), want):
+                    np.testing.assert_array_equal(dev.map_frame(frames[0], "channel." + ch)[0], x)
+    first, second, third = (float(np.median(t[4:])) for t in us)
+    print(f"[grid] frames of a build: {first:.1f}, {second:.1f}, {third:.1f} us", flush=True)
+    assert first > 1.04 * second and first > 1.04 * third
+    dev.commit(s.world)
+    scene = B.scene_of(dev, s.world)
+    vol = N.vrx_volume()
+    N.check(N.hip().vrx_memcpy_sync(C.addressof(vol), C.c_void_p(scene.d_volumes),
+                                    C.c_size_t(C.sizeof(vol)), N.VRX_D2H))
+    assert vol.d_majorant and vol.grid_format == 0x64737431
+    render(frames[0])
+    for ch, x in zip(("color", "depth", "objectId"), want):
+        np.testing.assert_array_equal(dev.map_frame(frames[0], "channel." + ch)[0], x)
+    assert not dev.errors(), dev.errors()
+    s.release()
+    dev.close()

@@ -297,8 +297,13 @@ struct World : Object {
   std::vector<vrx_geom> hostGeoms;
   uint64_t numPrims{0}; // of hostGeoms
   std::vector<Geometry *> hostGeomOf;
+  std::vector<vrx_volume> hostVolumes;
+  // grids wait for their distances; the build that frames have rendered
+  bool distancesPending{false};
+  uint64_t renderedBuild{0};
   int rebuild();
   int ensureWide(); // 4-wide nodes for every BLAS and the TLAS; sets scene.wide
+  void ensureGridDistances(); // distances behind the volumes' majorant grids
   void freeScene();
   bool needsRebuild() const;
 };

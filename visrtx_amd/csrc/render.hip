@@ -573,8 +573,8 @@ __global__ __launch_bounds__(256) void k_majorants(vrx_volume v, float *out)
 
 // One axis of the cells' Chebyshev distance to the nearest cell that is not
 // empty, min over the row of max(offset, the distance over the axes before);
-// AXIS 0 reads the majorants.  A few cells' loads per cell, once per world
-// build.
+// AXIS 0 reads the majorants.  A few cells' loads per cell, at most once per
+// world build.
 template <int AXIS>
 __global__ __launch_bounds__(256) void k_grid_distance(const float *majorant, const uint8_t *in,
     uint8_t *out, int mx, int my, int mz)
