@@ -88,11 +88,11 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(6, 8))) 
 // group's counter, each counter on a cache line of its own: one counter for
 // all waves serves an atomic in 11.4 ns, whatever a tile costs.  The groups
 // share every row of kTileCounters tiles in an order turned by one from row
-// to row, so that none is kept to some columns of the image.  (A grid of fewer
-// waves than counters has no more tiles than waves.)  1920x1080, AO of 1 spp
-// with one counter and with 32: 428 and 75 us for a frame that hits nothing,
-// 443 and 200 us for 500 spheres (41 and 193 us with a thread per pixel,
-// k_render_occ6); 64 counters are no faster.
+// to row, so that none is kept to some columns of the image.  A grid with a
+// wave for every tile (all that have fewer waves than counters) needs none of
+// this.  1920x1080, AO of 1 spp with one counter and with 32: 428 and 75 us
+// for a frame that hits nothing, 443 and 200 us for 500 spheres (41 and 193 us
+// with a thread per pixel, k_render_occ6); 64 counters are no faster.
 constexpr uint32_t kTileCounters = 32, kTileCounterWords = 32;
 
 // The counters start after the tiles that the waves start with.
@@ -133,8 +133,10 @@ k_render_sampled(vrx_scene sc, vrx_camera cam, vrx_renderer r, vrx_frame f, uint
       (uint32_t)__builtin_amdgcn_readfirstlane((int)(blockIdx.x * (kBlock / 64) + wave));
   const uint32_t g = id % kTileCounters;
   uint32_t *const counter = (uint32_t *)queues - (kTileCounters - g) * kTileCounterWords;
+  // with a wave for every tile each has the tile of its number alone
+  const bool deal = tiles > gridDim.x * (kBlock / 64);
   for (uint32_t k = id / kTileCounters;;) {
-    const uint32_t t = k * kTileCounters + (g + k) % kTileCounters;
+    const uint32_t t = deal ? k * kTileCounters + (g + k) % kTileCounters : id;
     if (t >= tiles)
       break;
     const uint32_t ty = t / tiles_x, tx = t - ty * tiles_x;
@@ -142,6 +144,8 @@ k_render_sampled(vrx_scene sc, vrx_camera cam, vrx_renderer r, vrx_frame f, uint
     const bool inside = px < f.width && py < f.height;
     render_wave<PT, TWO, KIND>(sc, cam, r, f, px, py, inside, (size_t)px + (size_t)py * f.width, st,
         q, rays);
+    if (!deal)
+      break;
     if (lane == 0)
       k = atomicAdd(counter, 1u);
     k = (uint32_t)__builtin_amdgcn_readfirstlane((int)k);
@@ -875,8 +879,9 @@ static void launch_one(const vrx_scene &sc, const vrx_camera &cam, const vrx_ren
       const uint32_t blocks = std::min(std::min((uint32_t)(per_cu * device_cus()),
           sampled_max_blocks(f.width, f.height)), (tx * ty + 3) / 4);
       uint32_t *counters = (uint32_t *)((char *)f.d_scratch + off);
-      hipLaunchKernelGGL(k_tile_counters, dim3(1), dim3(64), 0, s, counters,
-          blocks * (kBlock / 64));
+      if (tx * ty > blocks * (kBlock / 64))
+        hipLaunchKernelGGL(k_tile_counters, dim3(1), dim3(64), 0, s, counters,
+            blocks * (kBlock / 64));
       hipLaunchKernelGGL((k_render_sampled<PT, TWO, KIND>), dim3(blocks), dim3(kBlock), lds, s, sc,
           cam, r, f, sd, cap, (uint32_t *)f.d_scratch,
           (float *)(counters + kTileCounters * kTileCounterWords), tx, tx * ty);
