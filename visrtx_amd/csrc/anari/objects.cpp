@@ -1583,8 +1583,11 @@ int World::rebuild()
   memcpy(bounds, wb, sizeof(bounds));
   hostGeoms = std::move(hg);
   numPrims = 0;
-  for (const vrx_geom &g : hostGeoms)
+  opaque = true;
+  for (const vrx_geom &g : hostGeoms) {
     numPrims += g.n;
+    opaque = opaque && g.opacity == 1.0f;
+  }
   hostGeomOf = std::move(geomOf);
   hostVolumes = std::move(hv);
   distancesPending = nGrids > 0;
@@ -1938,6 +1941,10 @@ constexpr int kLongRaySteps = 32;
 // that no choice fits, and the first candidate, without the long-ray pass,
 // stays.
 constexpr float kTuneBand = 1.5f;
+// The launches that only suit frames with little to do are tried where a frame
+// is short (ms), and have to win by more than frames of one launch differ:
+// later candidates run on a warmer chip.
+constexpr float kTuneCheap = 2.0f, kTuneGain = 0.95f;
 constexpr uint32_t kTuneSoon = 32;
 
 bool Frame::rebuiltOff()
@@ -1953,7 +1960,7 @@ bool Frame::rebuiltOff()
   return __builtin_popcount(tune.off) >= 2;
 }
 
-void Frame::pickLaunch(vrx_renderer &rr)
+bool Frame::pickLaunch(vrx_renderer &rr)
 {
   // A rebuilt world keeps what its frames have measured: starting over with
   // every rebuild, it rendered with the first candidate for ever (131k
@@ -1978,13 +1985,7 @@ void Frame::pickLaunch(vrx_renderer &rr)
     tune.key = key;
     tune.hasty = hasty;
     // the first frame also pays for cold caches and page tables, so its stack
-    // depth is tried again last.  BVH2 nodes are not tried: the packed 4-wide
-    // nodes are faster on every scene measured (10M spheres 0.45 against
-    // 0.50 ms, AO 16 spp 10.8 against 14.2 ms, heightfield 0.15 against 0.18;
-    // and in the generic kernel, raycast, AO and directLight: 100k cones 0.65,
-    // 2.7, 3.3 against 0.81, 3.2, 4.0 ms, three primitive types of 300k each
-    // 1.8, 6.3, 7.7 against 2.2, 7.3, 9.3, 1M spheres and a 128^3 volume
-    // 0.52, 1.9, 2.5 against 0.68, 2.5, 3.2)
+    // depth is tried again last
     const int sds[3] = {16, 32, 16};
     const int ns = renderer->tuneStack ? 3 : 1;
     // the long-ray pass applies to one-level scenes of one primitive type;
@@ -1993,6 +1994,27 @@ void Frame::pickLaunch(vrx_renderer &rr)
     tune.deferPending = renderer->tuneDefer && world->scene.num_entries == 1
         && world->scene.num_volumes == 0
         && (st == VRX_TRIANGLE || st == VRX_SPHERE || st == VRX_CYLINDER);
+    // The ray queues of AO and directLight cost more than they bring where a
+    // hit sends few rays and few pixels hit (100k instances at 1 AO sample:
+    // 1.20 ms with them, 0.99 with a thread per pixel; 1M lit spheres 3.1
+    // against 3.8), so one frame is tried without.
+    tune.pixelPending = renderer->tuneWidth && rr.kind != VRX_RENDER_RAYCAST
+        && world->scene.num_volumes == 0
+        && (st == VRX_TRIANGLE || st == VRX_SPHERE || st == VRX_CYLINDER);
+    // Packed nodes are faster where rays walk far (10M spheres 0.45 against
+    // 0.50 ms, AO 16 spp 10.8 against 14.2 ms, heightfield 0.15 against 0.18;
+    // in the generic kernel, raycast, AO and directLight: 100k cones 0.65, 2.7,
+    // 3.3 against 0.81, 3.2, 4.0 ms, 1M spheres and a 128^3 volume 0.52, 1.9,
+    // 2.5 against 0.68, 2.5, 3.2), but their kernels hold more per lane, and
+    // frames that hit little are over sooner on BVH2 nodes (AO of 1 spp,
+    // 1920x1080: 41 against 75 us for a frame that hits nothing, 116 against
+    // 130 for 300 instances), so these are tried once.  Not where the frame
+    // could differ: any-hit walks add translucent surfaces in the order of the
+    // nodes, and in scaled instances the cylinder, cone and curve tests report
+    // hits off the primitive, which depend on it too.
+    tune.bvh2Pending = renderer->tuneWidth && world->scene.num_entries > 0
+        && (rr.kind == VRX_RENDER_RAYCAST || world->opaque)
+        && (st == VRX_TRIANGLE || st == VRX_SPHERE || world->instances.empty());
     for (int a = 0; a < ns; a++) {
       tune.width[tune.n] = renderer->tuneWidth ? 4 : rr.node_width;
       tune.sd[tune.n] = renderer->tuneStack ? sds[a] : rr.stack_lds;
@@ -2012,15 +2034,23 @@ void Frame::pickLaunch(vrx_renderer &rr)
     if (tune.next >= tune.n) {
       int b = 0;
       for (int i = 1; i < tune.n; i++)
-        if (tune.ms[i] < tune.ms[b])
+        if (tune.ms[i] < (tune.pixel[i] || tune.width[i] != tune.width[0] ? kTuneGain : 1.0f) * tune.ms[b])
           b = i;
-      if (tune.deferPending) {
-        // one more candidate: the fastest launch with the long-ray pass
+      if (!(tune.ms[b] < kTuneCheap))
+        tune.pixelPending = tune.bvh2Pending = false;
+      // one more candidate at a time, from the fastest so far
+      tune.width[tune.n] = tune.width[b];
+      tune.sd[tune.n] = tune.sd[b];
+      tune.defer[tune.n] = tune.defer[b];
+      if (tune.pixelPending) {
+        tune.pixelPending = false;
+        tune.pixel[tune.n++] = true;
+      } else if (tune.bvh2Pending) {
+        tune.bvh2Pending = false;
+        tune.width[tune.n++] = 2;
+      } else if (tune.deferPending) {
         tune.deferPending = false;
-        tune.width[tune.n] = tune.width[b];
-        tune.sd[tune.n] = tune.sd[b];
-        tune.defer[tune.n] = kLongRaySteps;
-        tune.n++;
+        tune.defer[tune.n++] = kLongRaySteps;
       } else {
         tune.best = b;
         tune.chosenBuild = tune.lastBuild;
@@ -2035,6 +2065,7 @@ void Frame::pickLaunch(vrx_renderer &rr)
   rr.node_width = tune.width[use];
   rr.stack_lds = tune.sd[use];
   rr.defer_steps = tune.defer[use];
+  return tune.pixel[use];
 }
 
 void Frame::render()
@@ -2075,7 +2106,7 @@ void Frame::render()
     frameID += (uint32_t)spp;
   }
   vrx_renderer rr = renderer->r;
-  pickLaunch(rr);
+  const bool pixel = pickLaunch(rr);
   if (rr.node_width == 4 && world->ensureWide() != 0)
     return;
   if (rr.skip_empty) {
@@ -2109,6 +2140,12 @@ void Frame::render()
   }
   f.d_scratch = dScratch;
   f.scratch_bytes = scratchBytes;
+  if (pixel) {
+    // scratch as for another renderer holds no ray queues
+    vrx_renderer raycast = rr;
+    raycast.kind = VRX_RENDER_RAYCAST;
+    f.scratch_bytes = vrx_render_scratch_bytes(&world->scene, &raycast, f.width, f.height);
+  }
   f.d_counters = (uint64_t *)dCounters;
   vrx_event_record(evStart, dev->stream);
   dev->check(vrx_render(&world->scene, &camera->cam, &rr, &f, dev->stream), this, "render");

@@ -296,6 +296,7 @@ struct World : Object {
   // host copies of the scene tables (for re-upload when 4-wide nodes appear)
   std::vector<vrx_geom> hostGeoms;
   uint64_t numPrims{0}; // of hostGeoms
+  bool opaque{true};    // all of them
   std::vector<Geometry *> hostGeomOf;
   std::vector<vrx_volume> hostVolumes;
   // grids wait for their distances; the build that frames have rendered
@@ -361,8 +362,8 @@ struct Frame : Object {
   bool rendered{false};
   bool stackReported{false};
   // Online launch autotuning: the first frames of a configuration each use one
-  // candidate (node width x LDS stack depth, then the long-ray pass), timed by
-  // the frame's events; then the fastest is kept.  Every candidate gives
+  // candidate (LDS stack depths on packed nodes, then AO and directLight without
+  // ray queues, BVH2 nodes, the long-ray pass), timed by the frame's events; then the fastest is kept.  Every candidate gives
   // bit-identical channels, so tuning only changes the time.
   struct Tune {
     // what the measurements belong to.  A world that is rebuilt with as many
@@ -385,7 +386,10 @@ struct Frame : Object {
     } key;
     int n{0}, next{0}, best{-1}, last{-1};
     bool deferPending{false}; // the long-ray candidate is still to be added
+    bool pixelPending{false}; // the candidate without ray queues is still to be added
+    bool bvh2Pending{false};  // the candidate on BVH2 nodes is still to be added
     int width[8]{}, sd[8]{}, defer[8]{};
+    bool pixel[8]{};          // a thread per pixel instead of the ray queues
     float ms[8]{};
     // frames of worlds rebuilt since the choice are watched (rebuiltOff())
     uint64_t chosenBuild{0}, lastBuild{0}; // the world's build at the choice, of the last frame
@@ -395,7 +399,7 @@ struct Frame : Object {
     bool settled{false};                   // no more choices for this key
   } tune;
   bool rebuiltOff();
-  void pickLaunch(vrx_renderer &rr);
+  bool pickLaunch(vrx_renderer &rr); // true: without ray queues
   // completion callbacks: each render with a callback posts one job; the
   // device's callback thread runs it and advances `sync`
   struct Sync {
